@@ -532,7 +532,8 @@ def routing_c5(torch, mxfp8gg, workloads, dev, steps=5, warmup=2):
 GEMM_SOURCE = ROOT / "mxfp8-grouped-gemm_amd" / "csrc" / "gemm.hip"
 # every file the GEMM translation unit includes from the tree, so an edit to a
 # shared device helper also marks a stored traffic figure stale
-GEMM_HEADERS = [ROOT / "mxfp8-grouped-gemm_amd" / "csrc" / "mx_device.h",
+GEMM_HEADERS = [ROOT / "mxfp8-grouped-gemm_amd" / "csrc" / "gemm_thin.h",
+                ROOT / "mxfp8-grouped-gemm_amd" / "csrc" / "mx_device.h",
                 ROOT / "mxfp8-grouped-gemm_amd" / "csrc" / "mxgg_internal.h",
                 ROOT / "include" / "mxgg.h"]
 TRAFFIC_FILE = ROOT / "profiles" / "traffic_grouped_fwd_c2.json"

@@ -32,6 +32,7 @@
 // taking a contiguous slice of every round.
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "mx_device.h"
@@ -44,6 +45,7 @@ constexpr int kTileP = 256;
 constexpr int kTileQ = 256;
 constexpr int kStageK = 128;    // contraction elements (bytes) per stage
 constexpr int kThreads = 256;
+constexpr int kWaves = kThreads / 64;
 constexpr uint32_t kOpBytes = 256u * kStageK;          // one operand of one stage: 32 KB
 constexpr uint32_t kScaleOff = 2u * kOpBytes;          // scale rows after P and Q data
 // Scale block b of a stage at kScaleOff + b * kScaleBlk: [P, Q][256] bytes and
@@ -411,8 +413,8 @@ __device__ __forceinline__ void release_barrier() {
 // them are loaded whole and the bytes outside are zeroed in registers right
 // after each fragment read.  Only experts whose token range is not a multiple
 // of 16 take this path.
-template <bool SCALED, bool MASK = false>
-__device__ __forceinline__ void mainloop(Smem& sm, const Operand& P, const Operand& Q,
+template <bool SCALED, bool MASK = false, class SM>
+__device__ __forceinline__ void mainloop(SM& sm, const Operand& P, const Operand& Q,
                                          uint32_t klo, uint32_t kend, v4f (&acc)[64]) {
   static_assert(!(SCALED && MASK), "a scale block cannot be split by a token mask");
 #pragma unroll
@@ -565,8 +567,8 @@ __device__ __forceinline__ uint32_t swap_lane_pair(uint32_t x) {
 // bank exactly twice.  The staging writes take the accumulators straight from
 // AGPRs.  The output is written once and not read again by the kernel, so the
 // row stores are nontemporal (measured faster, most for fp32 output).
-template <bool F32>
-__device__ __forceinline__ void epilogue(Smem& sm, const v4f (&acc)[64], char* out,
+template <bool F32, class SM>
+__device__ __forceinline__ void epilogue(SM& sm, const v4f (&acc)[64], char* out,
                                          int64_t ldo_bytes, uint32_t q0, uint32_t qbeg,
                                          uint32_t qend, uint32_t p0, uint32_t pend,
                                          bool accumulate = false) {
@@ -703,7 +705,8 @@ __device__ __forceinline__ void epilogue(Smem& sm, const v4f (&acc)[64], char* o
 // index) x 512 B (P index 0..255), 16-byte chunk k of row q at chunk
 // k ^ ((q / 4) mod 16): a half-wave writing one chunk column of 32 rows, or
 // reading one whole row, touches every bank at most twice.
-__device__ __forceinline__ void stage_bf16_tile(Smem& sm, const v4f (&acc)[64]) {
+template <class SM>
+__device__ __forceinline__ void stage_bf16_tile(SM& sm, const v4f (&acc)[64]) {
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = threadIdx.x >> 6;
   const uint32_t wp = wave & 1u, wq = wave >> 1;
@@ -737,7 +740,8 @@ __device__ __forceinline__ void stage_bf16_tile(Smem& sm, const v4f (&acc)[64]) 
 // bf16 output through the bf16 staging: wave w stores rows 64w .. 64w+63 of
 // the tile, two whole 512-byte rows per store instruction (lanes 0-31 one
 // row, 32-63 the next).
-__device__ __forceinline__ void epilogue_bf16(Smem& sm, const v4f (&acc)[64], char* out,
+template <class SM>
+__device__ __forceinline__ void epilogue_bf16(SM& sm, const v4f (&acc)[64], char* out,
                                               int64_t ldo_bytes, uint32_t q0, uint32_t qbeg,
                                               uint32_t qend, uint32_t p0, uint32_t pend) {
   stage_bf16_tile(sm, acc);
@@ -795,8 +799,8 @@ __device__ __forceinline__ void epilogue_bf16(Smem& sm, const v4f (&acc)[64], ch
 // KEEP: the bf16 gate and up values are also stored, as h[tok][pg + c] and
 // h[tok][F + pg + c] (ldh elements per row), for a backward that re-reads h:
 // the same bits epilogue_bf16 writes for the unfused projection.
-template <int MODE, bool KEEP>
-__device__ __forceinline__ void epilogue_swiglu(Smem& sm, const v4f (&acc)[64], uint8_t* aq,
+template <int MODE, bool KEEP, class SM>
+__device__ __forceinline__ void epilogue_swiglu(SM& sm, const v4f (&acc)[64], uint8_t* aq,
                                                 int64_t ldq, uint8_t* sc, int64_t s_row,
                                                 int64_t s_blk, uint32_t q0, uint32_t qbeg,
                                                 uint32_t qend, uint32_t pg, uint16_t* h,
@@ -1059,6 +1063,8 @@ __global__ __launch_bounds__(kThreads, 1) void k_grouped_fwd(FwdArgs args, uint3
     }
   }
 }
+
+#include "gemm_thin.h"
 
 // Sum of the split partials of the forward's last round, in split order (the
 // first partial is the starting value), stored inside the tile's group and
@@ -1389,7 +1395,17 @@ hipError_t launch_grouped_fwd(const FwdArgs& a, hipStream_t stream) {
                   : a.swiglu_mode == MXGG_SCALE_FLOOR ? (keep ? kOutSwigluKeepFloor : kOutSwigluFloor)
                   : a.out_f32                         ? kOutF32
                                                       : kOutBf16;
-#define MXGG_FWD(S, O) hipLaunchKernelGGL((k_grouped_fwd<S, O>), grid, block, 0, stream, a, gm)
+  // Thin tiles take experts of at most 64 rows.  The thin-capable kernel runs
+  // 256-row tiles up to 4% slower (its wide path shares registers with the thin
+  // one), so it is left out where the average expert has more rows than two
+  // thin tiles: 32 equal experts, N 4096, K 7168, this kernel against the other:
+  // 64 rows 179 / 190 us, 100 rows 194 / 194, 192 rows 212 / 204.
+  const bool thin = (int64_t)a.M <= 128 * (int64_t)(a.group_ends ? a.E : 1);
+#define MXGG_FWD(S, O)                                                                   \
+  if (thin)                                                                              \
+    hipLaunchKernelGGL((k_grouped_fwd_thin<S, O>), grid, block, 0, stream, a, gm);       \
+  else                                                                                   \
+    hipLaunchKernelGGL((k_grouped_fwd<S, O>), grid, block, 0, stream, a, gm)
 #define MXGG_FWD_OUT(S)                                           \
   switch (out) {                                                  \
     case kOutF32: MXGG_FWD(S, kOutF32); break;                    \

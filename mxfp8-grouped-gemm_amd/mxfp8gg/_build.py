@@ -18,7 +18,7 @@ BUILD_DIR = PKG_DIR.parent / "_build"
 LIB_PATH = PKG_DIR / "libmxgg.so"
 
 SOURCES = ["capi.hip", "quant.hip", "swiglu.hip", "route.hip", "groups.hip", "gemm.hip"]
-HEADERS = ["mxgg_internal.h", "mx_device.h"]
+HEADERS = ["mxgg_internal.h", "mx_device.h", "gemm_thin.h"]
 
 ARCH = os.environ.get("MXGG_OFFLOAD_ARCH", "gfx950")
 

@@ -1,0 +1,89 @@
+"""The grouped forward's thin tiles (experts of at most 64 rows).
+
+The launch takes the thin-capable kernel where the average expert has at most
+128 rows; the same groups inside a taller operand (rows past the last group
+end) take the 256-row kernel.  Every output element is the same chain of MFMAs
+in both, so the rows inside the groups must be equal bit for bit, and both are
+held against the float64 oracle.  K below, at and past the six ring stages
+makes the load stream cross tiles; N off the 128-column grid leaves a partial
+tile and an empty second half.
+"""
+import numpy as np
+import pytest
+import torch
+
+import mxfp8gg
+from mxfp8gg import ops
+from oracle import oracle as O
+from tests._helpers import assert_close_to_oracle, u8
+from tests.test_gpu_split import _rand_q
+
+pytestmark = pytest.mark.gpu
+
+SIZES = {
+    "thin": [64, 0, 1, 60, 3, 61, 2, 64],          # starts on and off the 4-row grid
+    "mixed": [5, 65, 64, 0, 128, 1, 300, 17],      # thin runs between wide tiles
+    "one": [33],
+}
+
+
+def _case(gpu, sizes, N, K, scaled, seed):
+    M, E = sum(sizes), len(sizes)
+    a, a_s = _rand_q((M, K), gpu, seed)
+    w, w_s = _rand_q((E, N, K), gpu, seed + 1)
+    ends = torch.tensor(np.cumsum(sizes), dtype=torch.int32, device=gpu)
+    return a, (a_s if scaled else None), w, (w_s if scaled else None), ends
+
+
+def _taller(a, a_s, E):
+    """The same rows in an operand of more than 128 rows per expert."""
+    rows = 128 * E + 1 + a.shape[0]
+    big = torch.zeros((rows, a.shape[1]), dtype=torch.uint8, device=a.device)
+    big[:a.shape[0]] = a.view(torch.uint8)
+    s = None
+    if a_s is not None:
+        s = torch.full((rows, a_s.shape[1]), 127, dtype=torch.uint8, device=a.device)
+        s[:a.shape[0]] = a_s
+    return big.view(a.dtype), s
+
+
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("scaled", [True, False])
+@pytest.mark.parametrize("sizes,N,K", [
+    ("thin", 128, 32), ("thin", 260, 640), ("thin", 136, 2080), ("mixed", 384, 768),
+    ("mixed", 100, 1056), ("one", 512, 896),
+])
+def test_thin_tiles_equal_wide_tiles(gpu, sizes, N, K, scaled, out_dtype):
+    sizes = SIZES[sizes]
+    a, a_s, w, w_s, ends = _case(gpu, sizes, N, K, scaled, 11)
+    y = ops.grouped_mm(a, w, ends, a_s, w_s, out_dtype=out_dtype, split_tail=False)
+    big, big_s = _taller(a, a_s, len(sizes))
+    wide = ops.grouped_mm(big, w, ends, big_s, w_s, out_dtype=out_dtype, split_tail=False)
+    bits = torch.int16 if out_dtype == torch.bfloat16 else torch.int32
+    assert torch.equal(y.view(bits), wide[:a.shape[0]].view(bits))
+    ref = O.grouped_fwd(u8(a), u8(a_s) if scaled else None, u8(w), u8(w_s) if scaled else None,
+                        np.cumsum(sizes))
+    assert_close_to_oracle(y, ref)
+
+
+@pytest.mark.parametrize("mode", ["rceil", "floor"])
+@pytest.mark.parametrize("sizes,F,K", [("thin", 128, 96), ("mixed", 256, 1024), ("one", 128, 800)])
+def test_thin_swiglu_equals_wide(gpu, sizes, F, K, mode):
+    sizes = SIZES[sizes]
+    g = torch.Generator(device=gpu).manual_seed(5)
+    M, E = sum(sizes), len(sizes)
+    x = torch.randn((M, K), generator=g, device=gpu).to(torch.bfloat16)
+    w = (torch.randn((E, 2 * F, K), generator=g, device=gpu) * 0.05).to(torch.bfloat16)
+    ends = torch.tensor(np.cumsum(sizes), dtype=torch.int32, device=gpu)
+    a, a_s = mxfp8gg.to_mxfp8_dim0(x, mode)
+    wq, ws = mxfp8gg.to_mxfp8_dim0(w, mode)
+    q, s, h = ops.grouped_mm_swiglu_quant(a, wq, ends, a_s, ws, mode, return_h=True)
+    q1, s1 = ops.grouped_mm_swiglu_quant(a, wq, ends, a_s, ws, mode)
+    big, big_s = _taller(a, a_s.contiguous(), E)
+    qw, sw, hw = ops.grouped_mm_swiglu_quant(big, wq, ends, big_s, ws, mode, return_h=True)
+    assert torch.equal(h.view(torch.int16), hw[:M].view(torch.int16))
+    for got in ((q, s), (q1, s1)):
+        assert torch.equal(got[0].view(torch.uint8), qw[:M].view(torch.uint8))
+        assert torch.equal(got[1], sw[:M])
+    aq, as_ = ops.swiglu_quant(h, mode)
+    assert torch.equal(q.view(torch.uint8), aq.view(torch.uint8)) and torch.equal(s, as_)
