@@ -432,10 +432,14 @@ __device__ __forceinline__ void mainloop(SM& sm, const Operand& P, const Operand
   st.template load_scale<0>(sm.ring[0], P, kbeg);
   st.template load_scale<1>(sm.ring[0], Q, kbeg);
   st.issue_data(sm.ring[0], P, Q, kbeg);
-  st.issue_data(sm.ring[1], P, Q, kbeg + kStageK);
-  st.template load_scale<0>(sm.ring[1], P, kbeg + kStageK);
-  st.template load_scale<1>(sm.ring[1], Q, kbeg + kStageK);
-  wait_barrier<SCALED ? 18 : 16>();
+  if (nst > 1) {
+    st.issue_data(sm.ring[1], P, Q, kbeg + kStageK);
+    st.template load_scale<0>(sm.ring[1], P, kbeg + kStageK);
+    st.template load_scale<1>(sm.ring[1], Q, kbeg + kStageK);
+    wait_barrier<SCALED ? 18 : 16>();
+  } else {
+    wait_barrier<0>();
+  }
   MXGG_FENCE();
   Frags f;
   KMask km;
@@ -457,17 +461,20 @@ __device__ __forceinline__ void mainloop(SM& sm, const Operand& P, const Operand
     read_sa<SCALED, 0>(r0, fa, f);
     read_sb<SCALED, 0>(r0, fa, f);
   }
-  // Past the last stage the loads fetch zeros into a slot nobody reads again,
-  // and the final reads fetch a stale slot that is never used, so the loop
-  // body has no branches.  nst >= 1 here (kend > klo); written as a do-while
-  // because a loop that may run zero times made the compiler zero the
-  // accumulators twice per tile, once for the zero-trip path.
+  // The final reads fetch a stale slot and are never used, so the stage body has
+  // no branches.  Two loops over it: the stages whose slot takes a later stage,
+  // then the last two (or fewer) without loads.  Loads past the end would fetch
+  // zeros, but each holds its wave's issue like any other: a weight gradient
+  // over 256 tokens is two stages, and 36 of its 72 loads were such (bf16 dW,
+  // 32 experts, N 7168, K 2048, 128 / 256 / 512 tokens each: 232 -> 216,
+  // 260 -> 250, 339 -> 321 us; contractions of 16 stages and more level).
   uint32_t s = 0;
-  do {
+  auto stage = [&](auto loads) __attribute__((always_inline)) {
+    constexpr bool LOADS = decltype(loads)::value;
     uint8_t* cur = sm.ring[s & 1u];
     uint8_t* nxt = sm.ring[(s & 1u) ^ 1u];
-    uint32_t bp, bq;
-    st.stage_base(kbeg + (s + 2) * kStageK, bp, bq);
+    uint32_t bp = 0, bq = 0;
+    if constexpr (LOADS) st.stage_base(kbeg + (s + 2) * kStageK, bp, bq);
       mma<0, 0>(f, acc); read_a<4>(cur, fa, f); MASKA(4); MXGG_FENCE();
       mma<0, 1>(f, acc); read_sa<SCALED, 1>(cur, fa, f); MXGG_FENCE();
       mma<0, 2>(f, acc); read_a<5>(cur, fa, f); MASKA(5); MXGG_FENCE();
@@ -482,62 +489,65 @@ __device__ __forceinline__ void mainloop(SM& sm, const Operand& P, const Operand
       mma<2, 3>(f, acc); MXGG_FENCE();
       release_barrier();
       MXGG_FENCE();
-      mma<3, 0>(f, acc); st.load_p(cur, P, bp, 0); MXGG_FENCE();
+      mma<3, 0>(f, acc); if constexpr (LOADS) st.load_p(cur, P, bp, 0); MXGG_FENCE();
       mma<3, 1>(f, acc); MXGG_FENCE();
       mma<3, 2>(f, acc); MXGG_FENCE();
-      mma<3, 3>(f, acc); st.load_p(cur, P, bp, 1); MXGG_FENCE();
+      mma<3, 3>(f, acc); if constexpr (LOADS) st.load_p(cur, P, bp, 1); MXGG_FENCE();
       mma<4, 0>(f, acc); MXGG_FENCE();
       mma<4, 1>(f, acc); MXGG_FENCE();
-      mma<4, 2>(f, acc); st.load_p(cur, P, bp, 2); MXGG_FENCE();
+      mma<4, 2>(f, acc); if constexpr (LOADS) st.load_p(cur, P, bp, 2); MXGG_FENCE();
       mma<4, 3>(f, acc); MXGG_FENCE();
       mma<5, 0>(f, acc); MXGG_FENCE();
-      mma<5, 1>(f, acc); st.load_p(cur, P, bp, 3); MXGG_FENCE();
+      mma<5, 1>(f, acc); if constexpr (LOADS) st.load_p(cur, P, bp, 3); MXGG_FENCE();
       mma<5, 2>(f, acc); MXGG_FENCE();
       mma<5, 3>(f, acc); MXGG_FENCE();
-      mma<6, 0>(f, acc); st.load_p(cur, P, bp, 4); MXGG_FENCE();
+      mma<6, 0>(f, acc); if constexpr (LOADS) st.load_p(cur, P, bp, 4); MXGG_FENCE();
       mma<6, 1>(f, acc); MXGG_FENCE();
       mma<6, 2>(f, acc); MXGG_FENCE();
-      mma<6, 3>(f, acc); st.load_p(cur, P, bp, 5); MXGG_FENCE();
+      mma<6, 3>(f, acc); if constexpr (LOADS) st.load_p(cur, P, bp, 5); MXGG_FENCE();
       mma<7, 0>(f, acc); MXGG_FENCE();
       mma<7, 1>(f, acc); MXGG_FENCE();
-      mma<7, 2>(f, acc); st.load_p(cur, P, bp, 6); MXGG_FENCE();
+      mma<7, 2>(f, acc); if constexpr (LOADS) st.load_p(cur, P, bp, 6); MXGG_FENCE();
       mma<7, 3>(f, acc); MXGG_FENCE();
-      wait_barrier<7>();
+      wait_barrier<LOADS ? 7 : 0>();
       MXGG_FENCE();
       if constexpr (MASK) k_mask(km, kbeg + (s + 1) * kStageK, klo, kend);
       mma<0, 4>(f, acc); MXGG_FENCE();
       mma<0, 5>(f, acc); read_b<0>(nxt, fa, f); MASKB(0); MXGG_FENCE();
-      mma<0, 6>(f, acc); st.load_p(cur, P, bp, 7); MXGG_FENCE();
+      mma<0, 6>(f, acc); if constexpr (LOADS) st.load_p(cur, P, bp, 7); MXGG_FENCE();
       mma<0, 7>(f, acc); MXGG_FENCE();
       mma<1, 4>(f, acc); read_a<0>(nxt, fa, f); MASKA(0); MXGG_FENCE();
-      mma<1, 5>(f, acc); st.load_q(cur, Q, bq, 0); MXGG_FENCE();
+      mma<1, 5>(f, acc); if constexpr (LOADS) st.load_q(cur, Q, bq, 0); MXGG_FENCE();
       mma<1, 6>(f, acc); MXGG_FENCE();
       mma<1, 7>(f, acc); read_b<1>(nxt, fa, f); MASKB(1); MXGG_FENCE();
-      mma<2, 4>(f, acc); st.load_q(cur, Q, bq, 1); MXGG_FENCE();
+      mma<2, 4>(f, acc); if constexpr (LOADS) st.load_q(cur, Q, bq, 1); MXGG_FENCE();
       mma<2, 5>(f, acc); read_a<1>(nxt, fa, f); MASKA(1); MXGG_FENCE();
       mma<2, 6>(f, acc); MXGG_FENCE();
-      mma<2, 7>(f, acc); st.load_q(cur, Q, bq, 2); MXGG_FENCE();
+      mma<2, 7>(f, acc); if constexpr (LOADS) st.load_q(cur, Q, bq, 2); MXGG_FENCE();
       mma<3, 4>(f, acc); MXGG_FENCE();
-      mma<3, 5>(f, acc); read_b<2>(nxt, fa, f); MASKB(2); st.load_q(cur, Q, bq, 3); MXGG_FENCE();
+      mma<3, 5>(f, acc); read_b<2>(nxt, fa, f); MASKB(2); if constexpr (LOADS) st.load_q(cur, Q, bq, 3); MXGG_FENCE();
       mma<3, 6>(f, acc); read_a<2>(nxt, fa, f); MASKA(2); MXGG_FENCE();
       mma<3, 7>(f, acc); MXGG_FENCE();
-      mma<4, 4>(f, acc); st.load_q(cur, Q, bq, 4); MXGG_FENCE();
+      mma<4, 4>(f, acc); if constexpr (LOADS) st.load_q(cur, Q, bq, 4); MXGG_FENCE();
       mma<4, 5>(f, acc); MXGG_FENCE();
       mma<4, 6>(f, acc); read_a<3>(nxt, fa, f); MASKA(3); MXGG_FENCE();
-      mma<4, 7>(f, acc); st.load_q(cur, Q, bq, 5); MXGG_FENCE();
+      mma<4, 7>(f, acc); if constexpr (LOADS) st.load_q(cur, Q, bq, 5); MXGG_FENCE();
       mma<5, 4>(f, acc); read_b<3>(nxt, fa, f); MASKB(3); MXGG_FENCE();
       mma<5, 5>(f, acc); MXGG_FENCE();
-      mma<5, 6>(f, acc); st.load_q(cur, Q, bq, 6); MXGG_FENCE();
+      mma<5, 6>(f, acc); if constexpr (LOADS) st.load_q(cur, Q, bq, 6); MXGG_FENCE();
       mma<5, 7>(f, acc); read_sb<SCALED, 0>(nxt, fa, f); MXGG_FENCE();
-      mma<6, 4>(f, acc); st.load_q(cur, Q, bq, 7); MXGG_FENCE();
+      mma<6, 4>(f, acc); if constexpr (LOADS) st.load_q(cur, Q, bq, 7); MXGG_FENCE();
       mma<6, 5>(f, acc); MXGG_FENCE();
       mma<6, 6>(f, acc); read_sa<SCALED, 0>(nxt, fa, f); MXGG_FENCE();
-      mma<6, 7>(f, acc); st.template load_scale<0>(cur, P, kbeg + (s + 2) * kStageK); MXGG_FENCE();
+      mma<6, 7>(f, acc); if constexpr (LOADS) st.template load_scale<0>(cur, P, kbeg + (s + 2) * kStageK); MXGG_FENCE();
       mma<7, 4>(f, acc); MXGG_FENCE();
       mma<7, 5>(f, acc); MXGG_FENCE();
-      mma<7, 6>(f, acc); st.template load_scale<1>(cur, Q, kbeg + (s + 2) * kStageK); MXGG_FENCE();
+      mma<7, 6>(f, acc); if constexpr (LOADS) st.template load_scale<1>(cur, Q, kbeg + (s + 2) * kStageK); MXGG_FENCE();
       mma<7, 7>(f, acc); MXGG_FENCE();
-  } while (++s < nst);
+  };
+  for (; s + 2 < nst; ++s) stage(std::true_type{});
+  do stage(std::false_type{});
+  while (++s < nst);
 #undef MASKA
 #undef MASKB
   // Drain the loads past the end before the next tile's prologue reuses the slots.
