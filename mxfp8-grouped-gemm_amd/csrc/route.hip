@@ -131,18 +131,20 @@ __device__ void plan_offsets(int32_t* hist, int nv, int E, int pad, int64_t cap,
     }
     padded = (cnt + pad - 1) / pad * pad;
   }
-  // exclusive scan of the padded sizes over experts
-  scan[tid] = padded;
-  __syncthreads();
-  for (int off = 1; off < kPlanThreads; off <<= 1) {
-    const int32_t add = tid >= off ? scan[tid - off] : 0;
-    __syncthreads();
-    scan[tid] += add;
-    __syncthreads();
+  // inclusive scan of the padded sizes over experts: lane shifts within a wave,
+  // then the totals of the waves before it
+  int32_t inc = padded;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int32_t below = __shfl_up(inc, off);
+    inc += (tid & 63) >= off ? below : 0;
   }
-  const int32_t start = scan[tid] - padded;
+  if ((tid & 63) == 63) scan[tid >> 6] = inc;
+  __syncthreads();
+  for (int w = 0; w < (tid >> 6); ++w) inc += scan[w];
+  const int32_t start = inc - padded;
   if (tid < E) {
-    ends[tid] = scan[tid];
+    ends[tid] = inc;
     counts[tid] = cnt;
     // each histogram's first row: the expert's start plus the counts before
     // it (8 loads issued before their 8 stores)
@@ -159,7 +161,7 @@ __device__ void plan_offsets(int32_t* hist, int nv, int E, int pad, int64_t cap,
     }
     for (int32_t r = start + cnt; r < start + padded; ++r) src[r] = -1;
   }
-  if (tid == E - 1) *total_s = scan[tid];
+  if (tid == E - 1) *total_s = inc;
   __syncthreads();
   for (int64_t r = (int64_t)*total_s + tid; r < cap; r += kPlanThreads) src[r] = -1;
 }
@@ -169,7 +171,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_route_plan(
     int32_t* __restrict__ perm, int32_t* __restrict__ src, int32_t* __restrict__ ends,
     int32_t* __restrict__ counts) {
   __shared__ int32_t hist[kPlanWaves * kMaxGroups];  // [wave][expert]
-  __shared__ int32_t scan[kPlanThreads];
+  __shared__ int32_t scan[kPlanWaves];
   __shared__ int32_t total_s;
   const int tid = threadIdx.x;
   const int w = tid >> 6;
@@ -218,7 +220,7 @@ __global__ __launch_bounds__(kPlanBlockThreads) void k_plan_count(
 __global__ __launch_bounds__(kPlanThreads) void k_plan_offsets(
     int32_t* __restrict__ ws, int nblocks, int E, int pad, int64_t cap,
     int32_t* __restrict__ src, int32_t* __restrict__ ends, int32_t* __restrict__ counts) {
-  __shared__ int32_t scan[kPlanThreads];
+  __shared__ int32_t scan[kPlanWaves];
   __shared__ int32_t total_s;
   plan_offsets(ws, nblocks, E, pad, cap, src, ends, counts, scan, &total_s);
 }
@@ -280,17 +282,20 @@ __global__ __launch_bounds__(256) void k_gather_rows(
 // Up to 8 slots per token: the slots' rows and factors are read once (they
 // are the same for the whole wave) and every chunk's 8 row loads go out
 // together; the sum stays in k order.  More slots take the general loop.
+// blockIdx.y takes `per` chunks of the row: with few tokens a row is spread over
+// several waves, since one wave's trips are a chain of load latencies.
 constexpr int kCombineSlots = 8;
 constexpr int kCombineChunks = 4;
 
 template <bool SCORES>
 __global__ __launch_bounds__(256) void k_combine(
     const uint16_t* __restrict__ y, int64_t ldy, int64_t yrows, const int32_t* __restrict__ perm,
-    const float* __restrict__ scores, int64_t tokens, int topk, int chunks,
+    const float* __restrict__ scores, int64_t tokens, int topk, int row_chunks, int per,
     uint16_t* __restrict__ out, int64_t ldo) {
   const int lane = threadIdx.x & 63;
   const int64_t t = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   if (t >= tokens) return;
+  const int first = (int)blockIdx.y * per, chunks = min(row_chunks, first + per);
   const int32_t* pt = perm + t * topk;
   uint16_t* o = out + t * ldo;
   if (topk <= kCombineSlots) {
@@ -304,7 +309,7 @@ __global__ __launch_bounds__(256) void k_combine(
     }
     // kCombineChunks chunks of every slot row per trip: their 32 loads go out
     // together (C5: 430 -> 416 us against one chunk per trip)
-    for (int c0 = lane; c0 < chunks; c0 += 64 * kCombineChunks) {
+    for (int c0 = first + lane; c0 < chunks; c0 += 64 * kCombineChunks) {
       uint4 v[kCombineChunks][kCombineSlots];
 #pragma unroll
       for (int u = 0; u < kCombineChunks; ++u) {
@@ -340,7 +345,7 @@ __global__ __launch_bounds__(256) void k_combine(
     }
     return;
   }
-  for (int c = lane; c < chunks; c += 64) {
+  for (int c = first + lane; c < chunks; c += 64) {
     float acc[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
@@ -454,13 +459,22 @@ hipError_t launch_combine(const uint16_t* y, int64_t ldy, int64_t yrows, const i
                           const float* scores, int64_t tokens, int topk, int64_t cols, uint16_t* out,
                           int64_t ldo, hipStream_t stream) {
   if (tokens == 0 || cols == 0) return hipSuccess;
-  const dim3 grid((unsigned)((tokens + 3) / 4));
+  // A row is split into whole trips of the kernel (kCombineChunks * 64 chunks)
+  // until the launch has this many waves (top-8 rows of 7168: 64 tokens 16.5 ->
+  // 6.3 us, 1000 tokens 32 -> 27, 1900 level; splitting a row of one trip only
+  // reads perm twice: 1000 rows of 1024, 7.5 -> 8.7).
+  constexpr int64_t kCombineWaves = 4096;
+  constexpr int kTrip = 64 * kCombineChunks;
+  const int chunks = (int)(cols / 8), trips = (chunks + kTrip - 1) / kTrip;
+  const int64_t want = std::max<int64_t>(1, std::min<int64_t>(trips, kCombineWaves / tokens));
+  const int per = (int)((trips + want - 1) / want) * kTrip;
+  const dim3 grid((unsigned)((tokens + 3) / 4), (unsigned)((chunks + per - 1) / per));
   if (scores != nullptr)
     hipLaunchKernelGGL((k_combine<true>), grid, dim3(256), 0, stream, y, ldy, yrows, perm, scores,
-                       tokens, topk, (int)(cols / 8), out, ldo);
+                       tokens, topk, chunks, per, out, ldo);
   else
     hipLaunchKernelGGL((k_combine<false>), grid, dim3(256), 0, stream, y, ldy, yrows, perm, scores,
-                       tokens, topk, (int)(cols / 8), out, ldo);
+                       tokens, topk, chunks, per, out, ldo);
   return hipGetLastError();
 }
 

@@ -197,6 +197,22 @@ def test_combine_matches_oracle(gpu, scaled, T, K, E, H):
     assert np.array_equal(bits(got), ref)
 
 
+@pytest.mark.parametrize("T", [1, 5, 1025])
+@pytest.mark.parametrize("K,E,H", [(8, 16, 2048), (8, 16, 2056), (3, 5, 7168), (9, 12, 4104)])
+def test_combine_of_split_rows(gpu, T, K, E, H):
+    # few tokens: a row is spread over workgroups in pieces of 2048 columns
+    g = torch.Generator(device=gpu).manual_seed(T + H)
+    idx = torch.randint(0, E + 1, (T, K), generator=g, device=gpu)   # some slots dropped
+    plan = mxfp8gg.route_plan(idx, E)
+    y = torch.randn((plan.rows, H), generator=g, device=gpu).to(torch.bfloat16)
+    sc = torch.rand((T, K), generator=g, device=gpu)
+    perm = plan.perm.cpu().numpy()
+    for scores in (sc, None):
+        got = mxfp8gg.combine(y, plan, scores)
+        ref = O.combine(bits(y), perm, K, sc.cpu().numpy() if scores is not None else None)
+        assert np.array_equal(bits(got), ref)
+
+
 def test_combine_inverts_gather_for_top1(gpu):
     T, E, H = 999, 7, 72
     idx = _idx(gpu, T, 1, E, 10)
