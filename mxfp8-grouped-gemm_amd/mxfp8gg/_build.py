@@ -1,4 +1,5 @@
-"""Build libmxgg.so (gfx950 HIP kernels + C ABI) in-tree with hipcc.
+"""Build libmxgg.so (gfx950 HIP kernels + C ABI) in-tree with hipcc, and the host
+module _mxgg_host.so (csrc/host.cpp) with g++.
 
 The shared library lands next to this file so that it travels with the
 source tree; nothing is installed into site-packages.
@@ -16,6 +17,7 @@ CSRC_DIR = PKG_DIR.parent / "csrc"
 INCLUDE_DIR = PKG_DIR.parent.parent / "include"
 BUILD_DIR = PKG_DIR.parent / "_build"
 LIB_PATH = PKG_DIR / "libmxgg.so"
+HOST_PATH = PKG_DIR / "_mxgg_host.so"
 
 SOURCES = ["capi.hip", "quant.hip", "swiglu.hip", "route.hip", "groups.hip", "gemm.hip"]
 HEADERS = ["mxgg_internal.h", "mx_device.h", "gemm_thin.h"]
@@ -53,8 +55,28 @@ def _run(cmd: list[str]) -> None:
         print(out)
 
 
+def _host_command(out: Path) -> list[str]:
+    """g++ command of the host module (csrc/host.cpp, a torch extension without device code)."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    includes = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"]]
+    libdirs = cpp_extension.library_paths()
+    return [
+        os.environ.get("CXX") or shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC",
+        "-shared", "-fvisibility=hidden", "-DTORCH_API_INCLUDE_EXTENSION_H",
+        f"-DTORCH_EXTENSION_NAME={HOST_PATH.name.split('.')[0]}",
+        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+        *[f"-isystem{d}" for d in includes], str(CSRC_DIR / "host.cpp"), "-o", str(out),
+        *[f"-L{d}" for d in libdirs], "-lc10", "-ltorch_cpu", "-ltorch", "-ltorch_python",
+    ]
+
+
 def build(verbose: bool = True) -> Path:
-    """Compile every HIP source for gfx950 and link libmxgg.so (always rebuilds)."""
+    """Compile every HIP source for gfx950, link libmxgg.so and build the host
+    module beside it (always rebuilds)."""
     BUILD_DIR.mkdir(parents=True, exist_ok=True)
     cc = hipcc()
     objs = []
@@ -63,8 +85,11 @@ def build(verbose: bool = True) -> Path:
         obj = BUILD_DIR / (Path(src).stem + ".o")
         objs.append(obj)
         cmds.append([cc, *HIPCC_FLAGS, "-c", str(CSRC_DIR / src), "-o", str(obj)])
+    host_tmp = HOST_PATH.with_suffix(".so.tmp")
+    cmds.append(_host_command(host_tmp))
     with _cf.ThreadPoolExecutor(max_workers=len(cmds)) as ex:
         list(ex.map(_run, cmds))
+    os.replace(host_tmp, HOST_PATH)
     tmp = LIB_PATH.with_suffix(".so.tmp")
     _run([cc, "-shared", "-fPIC", f"--offload-arch={ARCH}", *map(str, objs), "-o", str(tmp)])
     os.replace(tmp, LIB_PATH)

@@ -10,7 +10,10 @@ import ctypes
 import threading
 from pathlib import Path
 
+import torch  # noqa: F401  (its libraries back the native host module)
+
 LIB_PATH = Path(__file__).resolve().parent / "libmxgg.so"
+HOST_PATH = Path(__file__).resolve().parent / "_mxgg_host.so"
 
 # mxgg_status
 OK = 0
@@ -140,11 +143,36 @@ class MxggError(RuntimeError):
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
+_native = None
+
+
+def native():
+    """The native host path (csrc/host.cpp), loaded with the library: checks,
+    allocations and the library call of an op in one step, for the plain case
+    of its arguments."""
+    if _native is None:
+        load()
+    return _native
+
+
+def _load_native(lib: ctypes.CDLL):
+    import importlib.machinery
+    import importlib.util
+
+    if not HOST_PATH.exists():
+        raise RuntimeError(f"{HOST_PATH} is missing: build it first (mxfp8gg._build.build())")
+    loader = importlib.machinery.ExtensionFileLoader("_mxgg_host", str(HOST_PATH))
+    mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_mxgg_host", loader))
+    loader.exec_module(mod)
+    mod.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in SIGNATURES})
+    return mod
 
 
 def load() -> ctypes.CDLL:
     """Load libmxgg.so and attach argument types (idempotent)."""
-    global _lib
+    global _lib, _native
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib
@@ -161,6 +189,7 @@ def load() -> ctypes.CDLL:
         v = lib.mxgg_abi_version()
         if v != ABI_VERSION:
             raise RuntimeError(f"libmxgg ABI version {v}, expected {ABI_VERSION}")
+        _native = _load_native(lib)
         _lib = lib
         return lib
 

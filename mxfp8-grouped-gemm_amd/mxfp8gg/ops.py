@@ -15,6 +15,8 @@ Reference entry points mirrored here (all paths under the reference repo):
 """
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from . import _lib
@@ -28,8 +30,37 @@ _MODES = {"rceil": _lib.SCALE_RCEIL, "floor": _lib.SCALE_FLOOR}
 # ---------------------------------------------------------------------------
 # helpers
 # ---------------------------------------------------------------------------
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream_ptr(t: torch.Tensor) -> int:
+    """The current stream of t's device, as the raw handle (the Python Stream
+    object costs several times the read)."""
+    if _raw_stream is not None:
+        return _raw_stream(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream
+
+
+def _native(x, scaling_mode="rceil"):
+    """The native host path for an op on the device tensor x, or None where the
+    Python form decides (another device, an unusual mode: it converts or
+    raises)."""
+    if isinstance(x, torch.Tensor) and x.is_cuda and scaling_mode.__class__ is str \
+            and scaling_mode in _MODES:
+        return _lib.native()
+    return None
+
+
+def _tensors(*ts) -> bool:
+    """Every argument is a tensor or None (what the native host path takes)."""
+    return all(t is None or isinstance(t, torch.Tensor) for t in ts)
+
+
+def _took(r, what: str) -> bool:
+    """Whether the native host path took the call; raises on a library status."""
+    if r.__class__ is int:
+        _lib.check(r, what)
+    return r is not None
 
 
 def _need_gpu(t: torch.Tensor, name: str) -> None:
@@ -190,6 +221,10 @@ def offs_to_group_ends(offs: torch.Tensor, tokens: int, offs_kind: str = "auto")
 def zero_rows_past_groups(out: torch.Tensor, offs: torch.Tensor) -> torch.Tensor:
     """Set the rows of a row-major 2-D `out` past the last group end to zero
     (the rows no grouped GEMM writes), reading the ends on the device."""
+    host = _native(out)
+    if host is not None and isinstance(offs, torch.Tensor):
+        if _took(host.zero_rows(out, offs, _stream_ptr(out)), "zero_rows_past_groups"):
+            return out
     _need_gpu(out, "out")
     if out.dim() != 2 or out.stride(-1) != 1:
         raise ValueError("out must be a row-major 2-D tensor")
@@ -289,6 +324,11 @@ def to_mxfp8_dim0(x: torch.Tensor, scaling_mode="rceil", scale_layout: str = "bl
     conversion); "row": contiguous row-major scales, written so by the cast
     itself (what torchao's casts return; a GEMM call converts them).
     """
+    host = _native(x, scaling_mode)
+    if host is not None and scale_layout in ("block", "row"):
+        r = host.dim0(x, scale_layout == "block", _MODES[scaling_mode], _stream_ptr(x))
+        if _took(r, "quant_dim0"):
+            return r
     _need_gpu(x, "x")
     if x.dtype != torch.bfloat16:
         raise TypeError(f"x must be bfloat16, got {x.dtype}")
@@ -335,6 +375,14 @@ def padded_token_capacity(num_tokens: int, num_groups: int | None) -> int:
     return (num_tokens + 31 * num_groups + 127) // 128 * 128
 
 
+def _dim1_native(x, offs, scaling_mode, scale_layout="block", cap=0):
+    host = _native(x, scaling_mode)
+    if host is None or scale_layout not in ("block", "row") or not _tensors(offs):
+        return None
+    r = host.dim1(x, offs, scale_layout == "block", cap, _MODES[scaling_mode], _stream_ptr(x))
+    return r if _took(r, "quant_dim1") else None
+
+
 def to_mxfp8_dim1(x: torch.Tensor, offs: torch.Tensor | None = None, scaling_mode="rceil",
                   scale_layout: str = "block"):
     """Token-axis MXFP8 for the wgrad operands, written transposed.
@@ -348,6 +396,9 @@ def to_mxfp8_dim1(x: torch.Tensor, offs: torch.Tensor | None = None, scaling_mod
     view of block-major storage ([M_pad/32][C]) with scale_layout "block"
     (default), contiguous row-major with "row".
     """
+    r = _dim1_native(x, offs, scaling_mode, scale_layout)
+    if r is not None:
+        return r[0], r[1], _mark_ends(r[2])
     _need_gpu(x, "x")
     if x.dtype != torch.bfloat16 or x.dim() != 2:
         raise TypeError("x must be a 2-D bfloat16 tensor")
@@ -383,6 +434,14 @@ def to_mxfp8_dim1(x: torch.Tensor, offs: torch.Tensor | None = None, scaling_mod
     return qt, st, _mark_ends(ends_pad)
 
 
+def _dual_native(x, offs, scaling_mode, cap=0):
+    host = _native(x, scaling_mode)
+    if host is None or not _tensors(offs):
+        return None
+    r = host.dual(x, offs, cap, _MODES[scaling_mode], _stream_ptr(x))
+    return r if _took(r, "quant_dual") else None
+
+
 def to_mxfp8_dual(x: torch.Tensor, offs: torch.Tensor | None = None, scaling_mode="rceil"):
     """Both MXFP8 casts of x from one read of it: the row-wise cast of
     to_mxfp8_dim0 and the token-axis cast of to_mxfp8_dim1, for operands a
@@ -392,6 +451,9 @@ def to_mxfp8_dual(x: torch.Tensor, offs: torch.Tensor | None = None, scaling_mod
     device) or None.  Returns (q, s, qt, st, offs_pad) with q, s as
     to_mxfp8_dim0(x) (rows inside the groups) and qt, st, offs_pad as
     to_mxfp8_dim1(x, offs)."""
+    r = _dual_native(x, offs, scaling_mode)
+    if r is not None:
+        return r[0], r[1], r[2], r[3], _mark_ends(r[4])
     _need_gpu(x, "x")
     if x.dtype != torch.bfloat16 or x.dim() != 2 or x.shape[1] % 32 != 0:
         raise TypeError("x must be a 2-D bfloat16 tensor [M, C] with C % 32 == 0")
@@ -434,6 +496,14 @@ def _weight_t_views(qt: torch.Tensor, st: torch.Tensor, E: int, N: int, K: int):
     return wt, wts
 
 
+# Weights of at most this many elements are cast as one run of rows: N % 32 == 0,
+# so no block of 32 rows straddles two experts, and the group table (three small
+# launches, 6 us on the device and 15 on the host) is not needed.  The large
+# casts run faster with it all the same (32 x 4096 x 7168: 747 us with the table
+# and its launches, 768 without).
+_UNGROUPED_WEIGHT = 1 << 28
+
+
 def quant_weight_dual(w: torch.Tensor, scaling_mode="rceil"):
     """Both casts of expert weights W [E, N, K] from one read: returns
     ((wq, ws), (wt, wts)) equal to to_mxfp8_dim0(w) (forward operand, blocks
@@ -444,7 +514,12 @@ def quant_weight_dual(w: torch.Tensor, scaling_mode="rceil"):
     E, N, K = w.shape
     if N % 32 != 0:
         raise ValueError(f"N={N} must be a multiple of 32 for MXFP8 blocks along N")
-    q, s, qt, st, _ = to_mxfp8_dual(w.reshape(E * N, K), _expert_ends(E, N, w.device), scaling_mode)
+    w2 = w.reshape(E * N, K)
+    r = None
+    if w.numel() <= _UNGROUPED_WEIGHT:
+        r = _dual_native(w2, None, scaling_mode, padded_token_capacity(E * N, E))
+    q, s, qt, st, _ = r if r is not None else \
+        to_mxfp8_dual(w2, _expert_ends(E, N, w.device), scaling_mode)
     return (q.reshape(E, N, K), s.reshape(E, N, K // 32)), _weight_t_views(qt, st, E, N, K)
 
 
@@ -501,6 +576,12 @@ def swiglu_backward_quant(h: torch.Tensor, grad_a: torch.Tensor, offs: torch.Ten
     Scales are views of block-major storage, as to_mxfp8_dim0 / to_mxfp8_dim1
     return them; M_pad = padded_token_capacity(M, E).  Rows of dh_q past the
     last group end are not written."""
+    host = _native(h, scaling_mode)
+    if host is not None and not return_bf16 and grad_a is not None and _tensors(grad_a, offs):
+        r = host.swiglu_bwd(h, grad_a, offs, _MODES[scaling_mode], _stream_ptr(h))
+        if _took(r, "swiglu_bwd_quant"):
+            return {"dh_q": r[0], "dh_s": r[1], "dh_qt": r[2], "dh_st": r[3], "a_qt": r[4],
+                    "a_st": r[5], "offs_pad": _mark_ends(r[6])}
     _need_gpu(h, "h")
     h, gate, up, f = _gate_up(h)
     M = h.shape[0]
@@ -597,6 +678,17 @@ def _full_rounds(M: int, N: int, E: int, device) -> bool:
     return any(0 < (m * n_tiles) % units <= units // 2 for m in range(m_lo, m_hi + 1))
 
 
+@functools.lru_cache(maxsize=1024)
+def _split_bytes(M: int, N: int, E: int, device) -> int:
+    """Workspace bytes of the forward's split entry where grouped_mm takes it
+    by itself, 0 where it does not."""
+    if M == 0 or N == 0:
+        return 0
+    if _small_launch(M, N, E, device) or _full_rounds(M, N, E, device):
+        return _split_workspace_bytes(device)
+    return 0
+
+
 _MAX_OPERAND_BYTES = 0x7FFFFFF0   # the C ABI's bound on (rows - 1) * ld + K
 
 
@@ -635,6 +727,14 @@ def grouped_mm(a: torch.Tensor, w: torch.Tensor, offs: torch.Tensor | None,
     round at most half full (the kernel then splits that round only if it
     does); True: always take the split entry point; False: never.
     """
+    host = _native(a)
+    if host is not None and out is None and split_tail is None and isinstance(w, torch.Tensor) \
+            and w.dim() == 3 and a.dim() == 2 and _tensors(offs, a_scales, w_scales) \
+            and out_dtype in (torch.bfloat16, torch.float32):
+        r = host.mm(a, w, offs, a_scales, w_scales, out_dtype == torch.float32,
+                    _split_bytes(a.shape[0], w.shape[1], w.shape[0], a.device), _stream_ptr(a))
+        if _took(r, "grouped_fwd"):
+            return r
     _need_gpu(a, "a")
     _need_gpu(w, "w")
     if a.dim() != 2 or w.dim() != 3:
@@ -687,8 +787,7 @@ def grouped_mm(a: torch.Tensor, w: torch.Tensor, offs: torch.Tensor | None,
                 e.data_ptr() if e is not None else None, E,
                 m, N, K, out.data_ptr() + r0 * out.stride(0) * esz, out.stride(0),
                 _out_code(out_dtype))
-        split = (_small_launch(m, N, E, a.device) or _full_rounds(m, N, E, a.device)) \
-            if split_tail is None else split_tail
+        split = _split_bytes(m, N, E, a.device) > 0 if split_tail is None else split_tail
         if split and m > 0 and N > 0:
             ws = _split_workspace(a.device)
             _lib.check(lib.mxgg_grouped_fwd_split(*args, ws.data_ptr(), ws.numel(), stream),
@@ -719,6 +818,12 @@ def grouped_mm_swiglu_quant(a: torch.Tensor, w: torch.Tensor, offs: torch.Tensor
     (q, scales, h); rows of h past the last group end are zero.  The
     reference runs the gate and up GEMMs, eager SiLU * up and the fp8 cast
     separately (e2e_bench.py:56-61)."""
+    host = _native(a, scaling_mode)
+    if host is not None and isinstance(w, torch.Tensor) and _tensors(offs, a_scales, w_scales):
+        r = host.mm_swiglu(a, w, offs, a_scales, w_scales, _MODES[scaling_mode], bool(return_h),
+                           _stream_ptr(a))
+        if _took(r, "grouped_fwd_swiglu_quant"):
+            return r
     _need_gpu(a, "a")
     _need_gpu(w, "w")
     if a.dim() != 2 or w.dim() != 3:
@@ -808,10 +913,12 @@ def fwd_ge(x_fp8, w_fp8, BLOCK_M=256, BLOCK_N=256, BLOCK_K=128, NUM_WARPS=4, GRO
 # ---------------------------------------------------------------------------
 # wgrad grouped GEMM
 # ---------------------------------------------------------------------------
+@functools.lru_cache(maxsize=64)
 def _cu_count(device) -> int:
     return torch.cuda.get_device_properties(device).multi_processor_count
 
 
+@functools.lru_cache(maxsize=1024)
 def wgrad_split_tokens(M: int, N: int, K: int, E: int, cus: int) -> int:
     """Split-K chunk (tokens) for a weight-gradient call, from shapes only.
 
@@ -854,6 +961,17 @@ def grouped_wgrad(go: torch.Tensor, ia: torch.Tensor, offs: torch.Tensor,
     (mxgg_grouped_wgrad_split): deterministic, any output dtype, equal to the
     unsplit result up to fp32 summation order.
     """
+    host = _native(go)
+    if host is not None and out is None and split_tokens is None and isinstance(ia, torch.Tensor) \
+            and isinstance(offs, torch.Tensor) and go.dim() == 2 and ia.dim() == 2 \
+            and offs.dim() == 1 and _tensors(go_scales, ia_scales) \
+            and out_dtype in (torch.bfloat16, torch.float32) \
+            and wgrad_split_tokens(go.shape[1], go.shape[0], ia.shape[0], len(offs),
+                                   _cu_count(go.device)) == 0:
+        r = host.wgrad(go, ia, offs, go_scales, ia_scales, out_dtype == torch.float32,
+                       _stream_ptr(go))
+        if _took(r, "grouped_wgrad"):
+            return r
     _need_gpu(go, "go")
     _need_gpu(ia, "ia")
     if go.dim() != 2 or ia.dim() != 2:
@@ -1040,7 +1158,12 @@ def quant_weight_for_dgrad(w: torch.Tensor, scaling_mode="rceil"):
     E, N, K = w.shape
     if N % 32 != 0:
         raise ValueError(f"N={N} must be a multiple of 32 for MXFP8 blocks along N")
-    qt, st, _ = to_mxfp8_dim1(w.reshape(E * N, K), _expert_ends(E, N, w.device), scaling_mode)
+    w2 = w.reshape(E * N, K)
+    r = None
+    if w.numel() <= _UNGROUPED_WEIGHT:
+        r = _dim1_native(w2, None, scaling_mode, cap=padded_token_capacity(E * N, E))
+    qt, st, _ = r if r is not None else \
+        to_mxfp8_dim1(w2, _expert_ends(E, N, w.device), scaling_mode)
     return _weight_t_views(qt, st, E, N, K)
 
 

@@ -25,8 +25,8 @@ from typing import NamedTuple
 import torch
 
 from . import _lib, ops
-from .ops import (_FP8, _block_major_buffer, _mode, _need_gpu, _stream_ptr,
-                  padded_token_capacity)
+from .ops import (_FP8, _MODES, _block_major_buffer, _mode, _native, _need_gpu, _stream_ptr,
+                  _tensors, _took, padded_token_capacity)
 
 __all__ = ["RoutePlan", "route_plan", "gather_rows", "gather_to_mxfp8_dual",
            "gather_to_mxfp8_dim0", "combine", "combine_score_grad"]
@@ -145,6 +145,12 @@ def gather_to_mxfp8_dual(x: torch.Tensor, plan: RoutePlan, scaling_mode="rceil",
     """Both MXFP8 casts of the routed rows (gather_rows(x, plan, row_scale)),
     read straight from token order.  Returns (q, s, qt, st, offs_pad) like
     to_mxfp8_dual(gather_rows(x, plan, row_scale), plan.offs)."""
+    host = _native(x, scaling_mode)
+    if host is not None and _tensors(row_scale) and x.shape[0] == plan.tokens:
+        r = host.gather_dual(x, plan.src, plan.offs, plan.topk, row_scale, _MODES[scaling_mode],
+                             _stream_ptr(x))
+        if _took(r, "gather_quant_dual"):
+            return r
     _need_gpu(x, "x")
     if x.dtype != torch.bfloat16 or x.dim() != 2 or x.shape[1] % 32 != 0:
         raise TypeError("x must be a 2-D bfloat16 tensor [tokens, H] with H % 32 == 0")
@@ -175,6 +181,11 @@ def gather_to_mxfp8_dim0(x: torch.Tensor, plan: RoutePlan, scaling_mode="rceil")
     """The row-wise MXFP8 cast of the routed rows (gather_rows(x, plan)), read
     straight from token order: the expert input of a forward-only pass.
     Returns (q [plan.rows, H], s) like to_mxfp8_dim0(gather_rows(x, plan))."""
+    host = _native(x, scaling_mode)
+    if host is not None:
+        r = host.gather_dim0(x, plan.src, plan.topk, _MODES[scaling_mode], _stream_ptr(x))
+        if _took(r, "gather_quant_dim0"):
+            return r
     _need_gpu(x, "x")
     if x.dtype != torch.bfloat16 or x.dim() != 2 or x.shape[1] % 32 != 0:
         raise TypeError("x must be a 2-D bfloat16 tensor [tokens, H] with H % 32 == 0")
@@ -197,6 +208,11 @@ def combine(y: torch.Tensor, plan: RoutePlan, scores: torch.Tensor | None = None
     """Back to token order: out[t] = bf16(sum_k bf16(y[perm[t, k]] * scores[t, k]))
     with the sum in fp32 in k order; without scores the plain sum of the
     routed rows (the input gradient of the gather).  y: bf16 [plan.rows, H]."""
+    host = _native(y)
+    if host is not None and _tensors(scores):
+        r = host.combine(y, plan.perm, plan.tokens, plan.topk, scores, _stream_ptr(y))
+        if _took(r, "combine"):
+            return r
     _need_gpu(y, "y")
     if y.dtype != torch.bfloat16 or y.dim() != 2 or y.shape[1] % 8 != 0:
         raise TypeError("y must be a 2-D bfloat16 tensor [rows, H] with H % 8 == 0")

@@ -1,0 +1,159 @@
+"""The native host path of the Python entry points against their Python form.
+
+Every op is called with arguments in the plain layout the native path takes
+and the same values in forms it leaves to the Python code (other strides,
+offsets, int64 or host-side group ends): the results must be equal, with the
+same shapes, types and strides, and what the Python form refuses is refused.
+"""
+import numpy as np
+import pytest
+import torch
+
+import mxfp8gg
+from mxfp8gg import _lib, ops, routing
+
+pytestmark = pytest.mark.gpu
+
+
+class _Off:
+    """The native path switched off, op by op (every function declines)."""
+
+    def __getattr__(self, name):
+        return lambda *a: None
+
+
+def _both(monkeypatch, fn):
+    with monkeypatch.context() as m:
+        m.setattr(_lib, "_native", _Off())
+        slow = fn()
+    return fn(), slow
+
+
+def _same(a, b):
+    if isinstance(a, dict):
+        assert a.keys() == b.keys()
+        for k in a:
+            _same(a[k], b[k])
+    elif isinstance(a, (tuple, list)):
+        assert len(a) == len(b)
+        for x, y in zip(a, b):
+            _same(x, y)
+    elif a is None:
+        assert b is None
+    else:
+        assert type(a) is type(b) and a.dtype == b.dtype
+        assert a.shape == b.shape and a.stride() == b.stride() and a.device == b.device
+        u, v = (t.as_subclass(torch.Tensor).contiguous() for t in (a, b))
+        assert torch.equal(u.view(torch.uint8), v.view(torch.uint8))
+
+
+def _bf16(gpu, *shape, seed=0):
+    g = torch.Generator(device=gpu).manual_seed(seed)
+    return torch.randn(shape, generator=g, device=gpu).to(torch.bfloat16)
+
+
+SIZES = [[40, 0, 77, 33], [1], [0, 0, 65], [256, 256]]
+
+
+@pytest.mark.parametrize("sizes", SIZES)
+@pytest.mark.parametrize("mode", ["rceil", "floor"])
+def test_casts(gpu, monkeypatch, sizes, mode):
+    x = _bf16(gpu, sum(sizes), 96)
+    ends = torch.tensor(np.cumsum(sizes), dtype=torch.int32, device=gpu)
+    w = _bf16(gpu, len(sizes), 64, 96, seed=1)
+    strided = _bf16(gpu, sum(sizes), 104)[:, :96]          # rows at a stride of 104
+    for fn in (lambda: ops.to_mxfp8_dim0(x, mode), lambda: ops.to_mxfp8_dim0(x, mode, "row"),
+               lambda: ops.to_mxfp8_dim0(w, mode), lambda: ops.to_mxfp8_dim0(strided, mode),
+               lambda: ops.to_mxfp8_dim1(x, ends, mode), lambda: ops.to_mxfp8_dim1(x, None, mode),
+               lambda: ops.to_mxfp8_dim1(x, ends, mode, "row"),
+               lambda: ops.to_mxfp8_dim1(x, ends.long(), mode),
+               lambda: ops.to_mxfp8_dual(x, ends, mode), lambda: ops.to_mxfp8_dual(x, None, mode),
+               lambda: ops.to_mxfp8_dual(strided, ends, mode),
+               lambda: ops.quant_weight_dual(w, mode),
+               lambda: ops.quant_weight_for_dgrad(w, mode)):
+        _same(*_both(monkeypatch, fn))
+
+
+@pytest.mark.parametrize("sizes", SIZES)
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+def test_gemms(gpu, monkeypatch, sizes, out_dtype):
+    M, E, N, K = sum(sizes), len(sizes), 256, 128
+    ends = torch.tensor(np.cumsum(sizes), dtype=torch.int32, device=gpu)
+    a, a_s = ops.to_mxfp8_dim0(_bf16(gpu, M, K))
+    w, w_s = ops.to_mxfp8_dim0(_bf16(gpu, E, N, K, seed=1))
+    # int64 and [E + 1] ends, row-major scales and columns off the 4-grid are
+    # the Python form's
+    lead0 = torch.cat([ends.new_zeros(1), ends])
+    for fn in (lambda: ops.grouped_mm(a, w, ends, a_s, w_s, out_dtype=out_dtype),
+               lambda: ops.grouped_mm(a, w, ends.long(), a_s, w_s, out_dtype=out_dtype),
+               lambda: ops.grouped_mm(a, w, lead0, a_s, w_s, out_dtype=out_dtype),
+               lambda: ops.grouped_mm(a, w, ends, a_s.contiguous(), w_s, out_dtype=out_dtype),
+               lambda: ops.grouped_mm(a, w, ends, out_dtype=out_dtype),
+               lambda: ops.grouped_mm(a, w[:, :255], ends, a_s, w_s[:, :255],
+                                      out_dtype=out_dtype)):
+        _same(*_both(monkeypatch, fn))
+    for keep in (False, True):
+        _same(*_both(monkeypatch, lambda: ops.grouped_mm_swiglu_quant(a, w, ends, a_s, w_s,
+                                                                      return_h=keep)))
+    go, gos, pad = ops.to_mxfp8_dim1(_bf16(gpu, M, 96), ends)
+    ia, ias, _ = ops.to_mxfp8_dim1(_bf16(gpu, M, 64, seed=2), ends)
+    for fn in (lambda: ops.grouped_wgrad(go, ia, pad, gos, ias, out_dtype=out_dtype),
+               lambda: ops.grouped_wgrad(go, ia, pad.long(), gos, ias, out_dtype=out_dtype),
+               lambda: ops.grouped_wgrad(go, ia, pad, out_dtype=out_dtype),
+               lambda: ops.grouped_wgrad(go, ia[:63], pad, gos, ias[:63], out_dtype=out_dtype)):
+        _same(*_both(monkeypatch, fn))
+
+
+@pytest.mark.parametrize("sizes", SIZES)
+def test_activation_and_rows(gpu, monkeypatch, sizes):
+    M = sum(sizes)
+    ends = torch.tensor(np.cumsum(sizes), dtype=torch.int32, device=gpu)
+    h, da = _bf16(gpu, M, 128), _bf16(gpu, M, 64, seed=1)
+    for offs in (ends, ends.long(), None):
+        _same(*_both(monkeypatch, lambda: ops.swiglu_backward_quant(h, da, offs)))
+    out = _bf16(gpu, M + 5, 64)
+    _same(*_both(monkeypatch, lambda: ops.zero_rows_past_groups(out.clone(), ends)))
+
+
+@pytest.mark.parametrize("T,K,E", [(1, 1, 1), (37, 3, 5)])
+def test_routing(gpu, monkeypatch, T, K, E):
+    g = torch.Generator(device=gpu).manual_seed(3)
+    plan = routing.route_plan(torch.randint(0, E, (T, K), generator=g, device=gpu), E)
+    x, sc = _bf16(gpu, T, 64), torch.rand((T, K), generator=g, device=gpu)
+    y = _bf16(gpu, plan.rows, 64, seed=1)
+    n = int(plan.offs[-1])   # rows past the last group end are not written by the dual cast
+
+    def dual(**kw):
+        q, s, *rest = routing.gather_to_mxfp8_dual(x, plan, **kw)
+        assert q.shape[0] == s.shape[0] == plan.rows
+        return (q[:n], s[:n], *rest)
+
+    for fn in (dual, lambda: dual(row_scale=sc), lambda: dual(row_scale=sc.double()),
+               lambda: routing.gather_to_mxfp8_dim0(x, plan),
+               lambda: routing.combine(y, plan, sc), lambda: routing.combine(y, plan),
+               lambda: routing.combine(y, plan, sc.double())):
+        _same(*_both(monkeypatch, fn))
+
+
+def test_refusals_stay(gpu):
+    x = _bf16(gpu, 64, 64)
+    with pytest.raises(TypeError):
+        ops.to_mxfp8_dim0(x.float())
+    with pytest.raises(ValueError):
+        ops.to_mxfp8_dim0(_bf16(gpu, 4, 40))
+    with pytest.raises(ValueError):
+        ops.to_mxfp8_dim0(x, "nearest")
+    with pytest.raises(ValueError):
+        ops.to_mxfp8_dim0(x, scale_layout="other")
+    q, s = ops.to_mxfp8_dim0(x)
+    w, ws = ops.to_mxfp8_dim0(_bf16(gpu, 2, 32, 64))
+    with pytest.raises(ValueError):
+        ops.grouped_mm(q, w, None, s, ws)
+    with pytest.raises(ValueError):
+        ops.grouped_mm(q, w, torch.tensor([1, 2, 3, 4], dtype=torch.int32, device=gpu), s, ws)
+    with pytest.raises(ValueError):
+        ops.grouped_mm(q, w, torch.tensor([32, 64], dtype=torch.int32, device=gpu), s, None)
+    with pytest.raises(AssertionError):
+        ops.grouped_mm(q[:, :32], w, torch.tensor([32, 64], dtype=torch.int32, device=gpu))
+    with pytest.raises(ValueError):
+        mxfp8gg.zero_rows_past_groups(x[:, :3], torch.tensor([1], dtype=torch.int32, device=gpu))
