@@ -8,13 +8,17 @@
 // the kernels read them).  For anything else it returns None and touches
 // nothing: the caller then runs the Python form, which converts, splits or
 // raises.  A result is a tensor or a tuple; an int is a library status.
+// Like torch's own ops, the functions run without the GIL (an allocation or a
+// launch on a full queue can block) and raise torch's exceptions (a trainer
+// catches torch.OutOfMemoryError).
 //
 // Library functions are reached through addresses handed in once by bind(), so
 // this module does not link against libmxgg.so.
 #include <torch/extension.h>
 
 #include <optional>
-#include <string>
+#include <tuple>
+#include <variant>
 #include <vector>
 
 #include "../../include/mxgg.h"
@@ -89,28 +93,40 @@ Tensor rows_view(const Tensor& buf, int64_t rows) {
 void* vp(const Tensor& t) { return t.data_ptr(); }
 const void* cp(const Tensor& t) { return t.const_data_ptr(); }
 void* st(int64_t stream) { return reinterpret_cast<void*>(stream); }
-py::object none() { return py::none(); }
+
+using Result = std::variant<std::monostate, int, Tensor, std::tuple<Tensor, Tensor>,
+                            std::tuple<Tensor, Tensor, Tensor>,
+                            std::tuple<Tensor, Tensor, OptTensor>,
+                            std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor>,
+                            std::tuple<Tensor, Tensor, Tensor, Tensor, OptTensor>,
+                            std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, OptTensor>>;
+Result none() { return std::monostate{}; }
 
 // E8M0 scales [rows, nblk] (or [E, rows, nblk]) stored block-major, as the
 // library's casts return them; the conditions are the Python form's.
 int64_t readable(const Tensor& t) {
   return (int64_t)t.storage().nbytes() - t.storage_offset() * t.element_size();
 }
-bool scales_2d(const Tensor& s, int64_t rows, int64_t nblk) {
-  return plain(s) && s.element_size() == 1 && s.dim() == 2 && s.size(0) == rows &&
+bool scale_bytes(const Tensor& s, const Tensor& of) {
+  const auto d = s.scalar_type();
+  return plain(s) && s.device() == of.device() &&
+         (d == at::kByte || d == at::kFloat8_e8m0fnu || d == at::kFloat8_e4m3fn || d == at::kChar);
+}
+bool scales_2d(const Tensor& s, const Tensor& of, int64_t rows, int64_t nblk) {
+  return scale_bytes(s, of) && s.dim() == 2 && s.size(0) == rows &&
          s.size(1) == nblk && (s.stride(0) == 1 || rows == 1) && s.stride(1) >= rows &&
          s.stride(1) % 4 == 0 && aligned(cp(s), 4) &&
          readable(s) >= (nblk - 1) * s.stride(1) + (rows + 3) / 4 * 4;
 }
-bool scales_3d(const Tensor& s, int64_t E, int64_t rows, int64_t nblk) {
-  return plain(s) && s.element_size() == 1 && s.dim() == 3 && s.size(0) == E &&
+bool scales_3d(const Tensor& s, const Tensor& of, int64_t E, int64_t rows, int64_t nblk) {
+  return scale_bytes(s, of) && s.dim() == 3 && s.size(0) == E &&
          s.size(1) == rows && s.size(2) == nblk && (s.stride(1) == 1 || rows == 1) &&
          s.stride(2) % 4 == 0 && (E == 1 || s.stride(0) % 4 == 0) && aligned(cp(s), 4) &&
          s.stride(2) >= rows && (E == 1 || s.stride(0) >= rows) &&
          readable(s) >= (E - 1) * s.stride(0) + (nblk - 1) * s.stride(2) + (rows + 3) / 4 * 4;
 }
 
-py::object dim0(const Tensor& x, bool block, int mode, int64_t stream) {
+Result dim0(const Tensor& x, bool block, int mode, int64_t stream) {
   if (!plain(x) || x.scalar_type() != at::kBFloat16 || x.dim() < 1 || !x.is_contiguous() ||
       x.size(-1) % 32 != 0 || !aligned(cp(x), 16))
     return none();
@@ -138,12 +154,12 @@ py::object dim0(const Tensor& x, bool block, int mode, int64_t stream) {
   const int rc = lib.quant_dim0(cp(x), rows, K, K, vp(q), K, vp(s), lds,
                                 block ? MXGG_SCALES_BLOCK_MAJOR : MXGG_SCALES_ROW_MAJOR, mode,
                                 st(stream));
-  if (rc != MXGG_OK) return py::int_(rc);
-  return py::make_tuple(q, s);
+  if (rc != MXGG_OK) return rc;
+  return std::make_tuple(q, s);
 }
 
 // cap: columns of the token-axis cast, 0 = padded_capacity.
-py::object dim1(const Tensor& x, const OptTensor& ends, bool block, int64_t cap, int mode,
+Result dim1(const Tensor& x, const OptTensor& ends, bool block, int64_t cap, int mode,
                 int64_t stream) {
   if (!bf16_rows(x) || x.size(1) % 8 != 0 || !ends_ok(ends, x)) return none();
   const int64_t M = x.size(0), C = x.size(1), E = ends ? ends->numel() : 0;
@@ -156,11 +172,11 @@ py::object dim1(const Tensor& x, const OptTensor& ends, bool block, int64_t cap,
       cp(x), M, C, x.stride(0), ends_ptr(ends), E, cap, vp(qt), cap, vp(buf), buf.stride(0),
       block ? MXGG_SCALES_BLOCK_MAJOR : MXGG_SCALES_ROW_MAJOR,
       pad ? pad->data_ptr<int32_t>() : nullptr, mode, st(stream));
-  if (rc != MXGG_OK) return py::int_(rc);
-  return py::make_tuple(qt, block ? rows_view(buf, C) : buf, pad);
+  if (rc != MXGG_OK) return rc;
+  return std::make_tuple(qt, block ? rows_view(buf, C) : buf, pad);
 }
 
-py::object dual(const Tensor& x, const OptTensor& ends, int64_t cap, int mode, int64_t stream) {
+Result dual(const Tensor& x, const OptTensor& ends, int64_t cap, int mode, int64_t stream) {
   if (!bf16_rows(x) || x.size(1) % 32 != 0 || !ends_ok(ends, x)) return none();
   const int64_t M = x.size(0), C = x.size(1), E = ends ? ends->numel() : 0;
   if (cap == 0) cap = padded_capacity(M, E);
@@ -172,8 +188,8 @@ py::object dual(const Tensor& x, const OptTensor& ends, int64_t cap, int mode, i
                                 sb.stride(0), vp(qt), cap, vp(stb), stb.stride(0),
                                 MXGG_SCALES_BLOCK_MAJOR, pad ? pad->data_ptr<int32_t>() : nullptr,
                                 mode, st(stream));
-  if (rc != MXGG_OK) return py::int_(rc);
-  return py::make_tuple(q, rows_view(sb, M), qt, rows_view(stb, C), pad);
+  if (rc != MXGG_OK) return rc;
+  return std::make_tuple(q, rows_view(sb, M), qt, rows_view(stb, C), pad);
 }
 
 // Operands of the grouped forward, checked.
@@ -196,7 +212,7 @@ bool fwd_in(const Tensor& a, const Tensor& w, const OptTensor& ends, const OptTe
       (in.M - 1) * a.stride(0) + in.K > kMaxOperandBytes)
     return false;
   if (as) {
-    if (!scales_2d(*as, in.M, in.K / 32) || !scales_3d(*ws, in.E, in.N, in.K / 32)) return false;
+    if (!scales_2d(*as, a, in.M, in.K / 32) || !scales_3d(*ws, a, in.E, in.N, in.K / 32)) return false;
     in.as = cp(*as);
     in.ldas = as->stride(1);
     in.ws = cp(*ws);
@@ -207,7 +223,7 @@ bool fwd_in(const Tensor& a, const Tensor& w, const OptTensor& ends, const OptTe
 }
 
 // split: workspace bytes of the split entry, 0 for the unsplit one.
-py::object mm(const Tensor& a, const Tensor& w, const OptTensor& ends, const OptTensor& as,
+Result mm(const Tensor& a, const Tensor& w, const OptTensor& ends, const OptTensor& as,
               const OptTensor& ws, bool f32, int64_t split, int64_t stream) {
   FwdIn in;
   if (!fwd_in(a, w, ends, as, ws, in) || in.N % 4 != 0) return none();
@@ -224,11 +240,11 @@ py::object mm(const Tensor& a, const Tensor& w, const OptTensor& ends, const Opt
                          in.ws, in.wsg, in.ldws, ends_ptr(ends), in.E, in.M, in.N, in.K, vp(out),
                          in.N, type, st(stream));
   }
-  if (rc != MXGG_OK) return py::int_(rc);
-  return py::cast(out);
+  if (rc != MXGG_OK) return rc;
+  return out;
 }
 
-py::object mm_swiglu(const Tensor& a, const Tensor& w, const OptTensor& ends, const OptTensor& as,
+Result mm_swiglu(const Tensor& a, const Tensor& w, const OptTensor& ends, const OptTensor& as,
                      const OptTensor& ws, int mode, bool keep, int64_t stream) {
   FwdIn in;
   if (!fwd_in(a, w, ends, as, ws, in) || in.N % 256 != 0) return none();
@@ -252,13 +268,13 @@ py::object mm_swiglu(const Tensor& a, const Tensor& w, const OptTensor& ends, co
         in.ldws, ends_ptr(ends), in.E, in.M, F, in.K, vp(q), F, vp(buf), buf.stride(0),
         MXGG_SCALES_BLOCK_MAJOR, mode, st(stream));
   }
-  if (rc != MXGG_OK) return py::int_(rc);
-  return keep ? py::make_tuple(q, rows_view(buf, in.M), h)
-              : py::make_tuple(q, rows_view(buf, in.M));
+  if (rc != MXGG_OK) return rc;
+  if (keep) return std::make_tuple(q, rows_view(buf, in.M), h);
+  return std::make_tuple(q, rows_view(buf, in.M));
 }
 
 // Unsplit weight gradient into a new dW.
-py::object wgrad(const Tensor& go, const Tensor& ia, const Tensor& ends, const OptTensor& gs,
+Result wgrad(const Tensor& go, const Tensor& ia, const Tensor& ends, const OptTensor& gs,
                  const OptTensor& is, bool f32, int64_t stream) {
   if (!bytes(go) || !bytes(ia) || go.dim() != 2 || ia.dim() != 2 || go.stride(1) != 1 ||
       ia.stride(1) != 1 || go.size(1) != ia.size(1) || go.device() != ia.device() ||
@@ -268,17 +284,17 @@ py::object wgrad(const Tensor& go, const Tensor& ia, const Tensor& ends, const O
   if (K % 4 != 0 || M % 32 != 0 || (N - 1) * go.stride(0) + M > kMaxOperandBytes ||
       (K - 1) * ia.stride(0) + M > kMaxOperandBytes)
     return none();
-  if (gs && (!scales_2d(*gs, N, M / 32) || !scales_2d(*is, K, M / 32))) return none();
+  if (gs && (!scales_2d(*gs, go, N, M / 32) || !scales_2d(*is, go, K, M / 32))) return none();
   Tensor dw = empty({E, N, K}, go, f32 ? at::kFloat : at::kBFloat16);
   const int rc = lib.grouped_wgrad(
       cp(go), go.stride(0), gs ? cp(*gs) : nullptr, gs ? gs->stride(1) : 0, cp(ia), ia.stride(0),
       is ? cp(*is) : nullptr, is ? is->stride(1) : 0, ends.const_data_ptr<int32_t>(), E, M, N, K,
       vp(dw), f32 ? MXGG_OUT_F32 : MXGG_OUT_BF16, 0, st(stream));
-  if (rc != MXGG_OK) return py::int_(rc);
-  return py::cast(dw);
+  if (rc != MXGG_OK) return rc;
+  return dw;
 }
 
-py::object swiglu_bwd(const Tensor& h, const Tensor& da, const OptTensor& ends, int mode,
+Result swiglu_bwd(const Tensor& h, const Tensor& da, const OptTensor& ends, int mode,
                       int64_t stream) {
   if (!bf16_rows(h) || !bf16_rows(da) || h.size(1) % 64 != 0 || da.size(0) != h.size(0) ||
       da.size(1) != h.size(1) / 2 || !ends_ok(ends, h) || h.device() != da.device())
@@ -296,25 +312,28 @@ py::object swiglu_bwd(const Tensor& h, const Tensor& da, const OptTensor& ends, 
       vp(sb), sb.stride(0), vp(qt), cap, vp(stb), stb.stride(0), vp(at), cap, vp(atb),
       atb.stride(0), pad ? pad->data_ptr<int32_t>() : nullptr, nullptr, 2 * F,
       MXGG_SCALES_BLOCK_MAJOR, mode, st(stream));
-  if (rc != MXGG_OK) return py::int_(rc);
-  return py::make_tuple(q, rows_view(sb, M), qt, rows_view(stb, 2 * F), at, rows_view(atb, F), pad);
+  if (rc != MXGG_OK) return rc;
+  return std::make_tuple(q, rows_view(sb, M), qt, rows_view(stb, 2 * F), at, rows_view(atb, F), pad);
 }
 
-py::object zero_rows(const Tensor& out, const Tensor& ends, int64_t stream) {
+Result zero_rows(const Tensor& out, const Tensor& ends, int64_t stream) {
   if (!plain(out) || out.dim() != 2 || out.stride(1) != 1 || !ends_ok(ends, out)) return none();
   const int64_t e = out.element_size();
   const int rc = lib.zero_rows_past_groups(vp(out), out.size(0), out.size(1) * e, out.stride(0) * e,
                                            ends.const_data_ptr<int32_t>(), ends.numel(),
                                            st(stream));
-  return py::int_(rc);
+  return rc;
 }
 
 // Routing: src / perm / offs are a plan's tensors.
-py::object gather_dual(const Tensor& x, const Tensor& src, const Tensor& offs, int topk,
+bool row_scores(const Tensor& s, const Tensor& of, int64_t slots) {
+  return plain(s) && s.scalar_type() == at::kFloat && s.is_contiguous() && s.numel() == slots &&
+         s.device() == of.device();
+}
+Result gather_dual(const Tensor& x, const Tensor& src, const Tensor& offs, int topk,
                        const OptTensor& scale, int mode, int64_t stream) {
   if (!bf16_rows(x) || x.size(1) % 32 != 0 || !ends_ok(src, x) || !ends_ok(offs, x) ||
-      (scale && (!plain(*scale) || scale->scalar_type() != at::kFloat || !scale->is_contiguous() ||
-                 scale->numel() != x.size(0) * topk)))
+      (scale && !row_scores(*scale, x, x.size(0) * topk)))
     return none();
   const int64_t M = src.numel(), C = x.size(1), E = offs.numel(), cap = padded_capacity(M, E);
   Tensor q = empty({M, C}, x, at::kFloat8_e4m3fn), qt = empty({C, cap}, x, at::kFloat8_e4m3fn);
@@ -325,49 +344,48 @@ py::object gather_dual(const Tensor& x, const Tensor& src, const Tensor& offs, i
       scale ? scale->const_data_ptr<float>() : nullptr, M, offs.const_data_ptr<int32_t>(), E, cap,
       vp(q), C, vp(sb), sb.stride(0), vp(qt), cap, vp(stb), stb.stride(0),
       MXGG_SCALES_BLOCK_MAJOR, pad.data_ptr<int32_t>(), mode, st(stream));
-  if (rc != MXGG_OK) return py::int_(rc);
-  return py::make_tuple(q, rows_view(sb, M), qt, rows_view(stb, C), pad);
+  if (rc != MXGG_OK) return rc;
+  return std::make_tuple(q, rows_view(sb, M), qt, rows_view(stb, C), pad);
 }
 
-py::object gather_dim0(const Tensor& x, const Tensor& src, int topk, int mode, int64_t stream) {
+Result gather_dim0(const Tensor& x, const Tensor& src, int topk, int mode, int64_t stream) {
   if (!bf16_rows(x) || x.size(1) % 32 != 0 || !ends_ok(src, x)) return none();
   const int64_t M = src.numel(), C = x.size(1);
   Tensor q = empty({M, C}, x, at::kFloat8_e4m3fn), sb = block_major(M, C / 32, x);
   const int rc = lib.gather_quant_dim0(cp(x), x.size(0), C, x.stride(0),
                                        src.const_data_ptr<int32_t>(), topk, M, vp(q), C, vp(sb),
                                        sb.stride(0), MXGG_SCALES_BLOCK_MAJOR, mode, st(stream));
-  if (rc != MXGG_OK) return py::int_(rc);
-  return py::make_tuple(q, rows_view(sb, M));
+  if (rc != MXGG_OK) return rc;
+  return std::make_tuple(q, rows_view(sb, M));
 }
 
-py::object combine(const Tensor& y, const Tensor& perm, int64_t tokens, int topk,
+Result combine(const Tensor& y, const Tensor& perm, int64_t tokens, int topk,
                    const OptTensor& scores, int64_t stream) {
   if (!bf16_rows(y) || y.size(1) % 8 != 0 || !ends_ok(perm, y) || perm.numel() != tokens * topk ||
-      (scores && (!plain(*scores) || scores->scalar_type() != at::kFloat ||
-                  !scores->is_contiguous() || scores->numel() != tokens * topk)))
+      (scores && !row_scores(*scores, y, tokens * topk)))
     return none();
   Tensor out = empty({tokens, y.size(1)}, y, at::kBFloat16);
   const int rc = lib.combine(cp(y), y.size(0), y.size(1), y.stride(0),
                              perm.const_data_ptr<int32_t>(),
                              scores ? scores->const_data_ptr<float>() : nullptr, tokens, topk,
                              vp(out), out.stride(0), st(stream));
-  if (rc != MXGG_OK) return py::int_(rc);
-  return py::cast(out);
+  if (rc != MXGG_OK) return rc;
+  return out;
 }
 
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("bind", &bind);
-  m.def("dim0", &dim0);
-  m.def("dim1", &dim1);
-  m.def("dual", &dual);
-  m.def("mm", &mm);
-  m.def("mm_swiglu", &mm_swiglu);
-  m.def("wgrad", &wgrad);
-  m.def("swiglu_bwd", &swiglu_bwd);
-  m.def("zero_rows", &zero_rows);
-  m.def("gather_dual", &gather_dual);
-  m.def("gather_dim0", &gather_dim0);
-  m.def("combine", &combine);
+  m.def("dim0", torch::wrap_pybind_function_no_gil(&dim0));
+  m.def("dim1", torch::wrap_pybind_function_no_gil(&dim1));
+  m.def("dual", torch::wrap_pybind_function_no_gil(&dual));
+  m.def("mm", torch::wrap_pybind_function_no_gil(&mm));
+  m.def("mm_swiglu", torch::wrap_pybind_function_no_gil(&mm_swiglu));
+  m.def("wgrad", torch::wrap_pybind_function_no_gil(&wgrad));
+  m.def("swiglu_bwd", torch::wrap_pybind_function_no_gil(&swiglu_bwd));
+  m.def("zero_rows", torch::wrap_pybind_function_no_gil(&zero_rows));
+  m.def("gather_dual", torch::wrap_pybind_function_no_gil(&gather_dual));
+  m.def("gather_dim0", torch::wrap_pybind_function_no_gil(&gather_dim0));
+  m.def("combine", torch::wrap_pybind_function_no_gil(&combine));
 }

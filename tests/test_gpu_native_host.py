@@ -23,6 +23,7 @@ class _Off:
 
 
 def _both(monkeypatch, fn):
+    assert _lib.native() is not None   # loaded before it is switched off and put back
     with monkeypatch.context() as m:
         m.setattr(_lib, "_native", _Off())
         slow = fn()
@@ -135,6 +136,38 @@ def test_routing(gpu, monkeypatch, T, K, E):
         _same(*_both(monkeypatch, fn))
 
 
+class _Log:
+    """The native path, noting which functions took their call."""
+
+    def __init__(self, real):
+        self.real, self.took = real, []
+
+    def __getattr__(self, name):
+        def call(*a):
+            r = getattr(self.real, name)(*a)
+            self.took.append((name, r is not None))
+            return r
+        return call
+
+
+def test_plain_forms_are_taken(gpu, monkeypatch):
+    """A small routed layer's training step and its parts run natively."""
+    log = _Log(_lib.native())
+    monkeypatch.setattr(_lib, "_native", log)
+    x, wgu, wd = _bf16(gpu, 64, 128), _bf16(gpu, 4, 256, 128), _bf16(gpu, 4, 128, 128)
+    idx = torch.arange(128, device=gpu, dtype=torch.int32).reshape(64, 2) % 4
+    leaves = [t.requires_grad_(True) for t in (x, wgu, wd)]
+    out = mxfp8gg.moe_routed_ffn(x, idx, None, wgu, wd)
+    torch.autograd.grad(out, leaves, torch.ones_like(out))
+    with torch.no_grad():
+        mxfp8gg.moe_routed_ffn(x, idx, None, wgu, wd)
+    ops.to_mxfp8_dim1(x.detach(), None)
+    ops.zero_rows_past_groups(out.detach(), torch.tensor([64], dtype=torch.int32, device=gpu))
+    assert all(t for _, t in log.took), log.took
+    assert {n for n, _ in log.took} == {"gather_dual", "gather_dim0", "dual", "dim0", "dim1", "mm",
+                                        "mm_swiglu", "wgrad", "swiglu_bwd", "combine", "zero_rows"}
+
+
 def test_refusals_stay(gpu):
     x = _bf16(gpu, 64, 64)
     with pytest.raises(TypeError):
@@ -157,3 +190,21 @@ def test_refusals_stay(gpu):
         ops.grouped_mm(q[:, :32], w, torch.tensor([32, 64], dtype=torch.int32, device=gpu))
     with pytest.raises(ValueError):
         mxfp8gg.zero_rows_past_groups(x[:, :3], torch.tensor([1], dtype=torch.int32, device=gpu))
+
+
+def test_scale_types_and_torch_errors(gpu):
+    """Scales of a type the Python form refuses are refused, those it takes are
+    read alike, and a failed allocation raises torch's own exception."""
+    ends = torch.tensor([32, 64], dtype=torch.int32, device=gpu)
+    q, s = ops.to_mxfp8_dim0(_bf16(gpu, 64, 64))
+    w, ws = ops.to_mxfp8_dim0(_bf16(gpu, 2, 32, 64))
+    for bad in (torch.float8_e5m2, torch.bool):
+        with pytest.raises(TypeError):
+            ops.grouped_mm(q, w, ends, s.view(bad), ws)
+        with pytest.raises(TypeError):
+            ops.grouped_mm(q, w, ends, s, ws.view(bad))
+    want = ops.grouped_mm(q, w, ends, s, ws)
+    for same in (torch.int8, torch.float8_e8m0fnu):
+        _same(ops.grouped_mm(q, w, ends, s.view(same), ws.view(same)), want)
+    with pytest.raises(torch.OutOfMemoryError):
+        ops._dim1_native(_bf16(gpu, 64, 64), None, "rceil", cap=1 << 46)
