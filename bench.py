@@ -533,6 +533,7 @@ GEMM_SOURCE = ROOT / "mxfp8-grouped-gemm_amd" / "csrc" / "gemm.hip"
 # every file the GEMM translation unit includes from the tree, so an edit to a
 # shared device helper also marks a stored traffic figure stale
 GEMM_HEADERS = [ROOT / "mxfp8-grouped-gemm_amd" / "csrc" / "gemm_thin.h",
+                ROOT / "mxfp8-grouped-gemm_amd" / "csrc" / "wgrad_ahead.h",
                 ROOT / "mxfp8-grouped-gemm_amd" / "csrc" / "mx_device.h",
                 ROOT / "mxfp8-grouped-gemm_amd" / "csrc" / "mxgg_internal.h",
                 ROOT / "include" / "mxgg.h"]

@@ -69,6 +69,9 @@ constexpr int64_t kPartialBytes = 256 * 256 * 4;
 // band width, then (expert, first item, chunks) of every rank; partial of
 // work item i at kWgHdrBytes + i * kPartialBytes.
 constexpr int64_t kWgHdrBytes = 32768;
+// Store instructions of one wave for a tile that lies inside dW, in the weight
+// gradient whose stores overlap the next tile (two per P half and Q fragment).
+constexpr int kAheadStores = 32;
 
 struct __align__(16) Smem {
   uint8_t ring[2][kStageBytes];
@@ -254,6 +257,19 @@ struct Stream {
            ok ? blk * X.lds : kOobOffset);
   }
 
+  // The loads of a tile's first two stages (18 each with scales), stage 0 first.
+  __device__ __forceinline__ void prologue(uint8_t* s0, uint8_t* s1, const Operand& P,
+                                           const Operand& Q, uint32_t kbeg, uint32_t nst) const {
+    load_scale<0>(s0, P, kbeg);
+    load_scale<1>(s0, Q, kbeg);
+    issue_data(s0, P, Q, kbeg);
+    if (nst > 1) {
+      issue_data(s1, P, Q, kbeg + kStageK);
+      load_scale<0>(s1, P, kbeg + kStageK);
+      load_scale<1>(s1, Q, kbeg + kStageK);
+    }
+  }
+
   // The 16 data loads of one stage, back to back (prologue only).
   __device__ __forceinline__ void issue_data(uint8_t* stage, const Operand& P, const Operand& Q,
                                              uint32_t k0) const {
@@ -413,10 +429,15 @@ __device__ __forceinline__ void release_barrier() {
 // them are loaded whole and the bytes outside are zeroed in registers right
 // after each fragment read.  Only experts whose token range is not a multiple
 // of 16 take this path.
-template <bool SCALED, bool MASK = false, class SM>
+// AHEAD (scaled only): the caller issued the loads of the first two stages
+// itself (issue_ahead()), then at most kAheadStores stores of the tile before,
+// or waited for all of it.  vmcnt retires in issue order, so the first waits
+// leave those stores in flight: they drain behind this tile's first two stages.
+template <bool SCALED, bool MASK = false, bool AHEAD = false, class SM>
 __device__ __forceinline__ void mainloop(SM& sm, const Operand& P, const Operand& Q,
                                          uint32_t klo, uint32_t kend, v4f (&acc)[64]) {
   static_assert(!(SCALED && MASK), "a scale block cannot be split by a token mask");
+  static_assert(SCALED || !AHEAD, "the wait counts of AHEAD include the scale loads");
 #pragma unroll
   for (int i = 0; i < 64; ++i) acc[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
   if (kend <= klo) return;
@@ -429,17 +450,12 @@ __device__ __forceinline__ void mainloop(SM& sm, const Operand& P, const Operand
   // Prologue: all of stage 0 and the data of stage 1 (its scales follow in
   // the first stage), then publish stage 0 and read the part of it that the
   // loop reads one stage ahead.
-  st.template load_scale<0>(sm.ring[0], P, kbeg);
-  st.template load_scale<1>(sm.ring[0], Q, kbeg);
-  st.issue_data(sm.ring[0], P, Q, kbeg);
-  if (nst > 1) {
-    st.issue_data(sm.ring[1], P, Q, kbeg + kStageK);
-    st.template load_scale<0>(sm.ring[1], P, kbeg + kStageK);
-    st.template load_scale<1>(sm.ring[1], Q, kbeg + kStageK);
-    wait_barrier<SCALED ? 18 : 16>();
-  } else {
-    wait_barrier<0>();
-  }
+  if constexpr (!AHEAD) st.prologue(sm.ring[0], sm.ring[1], P, Q, kbeg, nst);
+  constexpr int kLeft = AHEAD ? kAheadStores : 0;
+  if (nst > 1)
+    wait_barrier<(SCALED ? 18 : 16) + kLeft>();
+  else
+    wait_barrier<kLeft>();
   MXGG_FENCE();
   Frags f;
   KMask km;
@@ -509,7 +525,10 @@ __device__ __forceinline__ void mainloop(SM& sm, const Operand& P, const Operand
       mma<7, 1>(f, acc); MXGG_FENCE();
       mma<7, 2>(f, acc); if constexpr (LOADS) st.load_p(cur, P, bp, 6); MXGG_FENCE();
       mma<7, 3>(f, acc); MXGG_FENCE();
-      wait_barrier<LOADS ? 7 : 0>();
+      if (AHEAD && (LOADS ? s == 0 : nst <= 2))
+        wait_barrier<(LOADS ? 7 : 0) + kLeft>();
+      else
+        wait_barrier<LOADS ? 7 : 0>();
       MXGG_FENCE();
       if constexpr (MASK) k_mask(km, kbeg + (s + 1) * kStageK, klo, kend);
       mma<0, 4>(f, acc); MXGG_FENCE();
@@ -550,8 +569,9 @@ __device__ __forceinline__ void mainloop(SM& sm, const Operand& P, const Operand
   while (++s < nst);
 #undef MASKA
 #undef MASKB
-  // Drain the loads past the end before the next tile's prologue reuses the slots.
-  wait_barrier<0>();
+  // Every wave has read its last fragments, and its loads have landed (the last
+  // publish wait), before the next tile's loads reuse the slots.
+  release_barrier();
 }
 
 #undef MXGG_FENCE
@@ -1280,6 +1300,8 @@ __global__ __launch_bounds__(kThreads, 1) void k_grouped_wgrad(WgradArgs args, u
   }
 }
 
+#include "wgrad_ahead.h"
+
 // dW tiles of experts whose tokens were cut into several chunks: the chunks'
 // fp32 partials added in chunk order (the first is the starting value);
 // experts without tokens (no work items) written as zeros; experts with one
@@ -1445,7 +1467,22 @@ hipError_t launch_grouped_wgrad(const WgradArgs& a, hipStream_t stream) {
   const dim3 grid(persistent_grid()), block(kThreads);
   const uint32_t gm = 4;
 #define MXGG_WG(S, F) hipLaunchKernelGGL((k_grouped_wgrad<S, F>), grid, block, 0, stream, a, gm)
-  if (a.scaled) {
+  // Up to 768 tokens per expert (M counts the padding) the tiles whose stores
+  // overlap the next tile's loads are faster, above they are level to 3%
+  // slower (a tile's store is then a small part of it, and the MFMAs of other
+  // CUs cover it).  32 experts, bf16 dW, k_grouped_wgrad against
+  // k_grouped_wgrad_ahead, us, tokens per expert:
+  //                      32       128       250       512        1000       2048
+  //   7168 x 2048   216/166   218/166   254/211   331/286    539/555    831/848
+  //   4096 x 7168   378/316   431/324   506/421   654/573  1062/1001  1630/1583
+  // dW rows off the 16-byte grid would all take the guarded stores.
+  constexpr int64_t kAheadTokens = 768;
+  const bool ahead = a.scaled && !a.out_f32 && a.split <= 0 &&
+                     ((a.ldw_n | a.ldw_e) & 7) == 0 &&
+                     (int64_t)a.M <= kAheadTokens * (int64_t)a.E;
+  if (ahead) {
+    hipLaunchKernelGGL(k_grouped_wgrad_ahead, grid, block, 0, stream, a, gm);
+  } else if (a.scaled) {
     if (a.out_f32) MXGG_WG(true, true); else MXGG_WG(true, false);
   } else {
     if (a.out_f32) MXGG_WG(false, true); else MXGG_WG(false, false);

@@ -20,7 +20,7 @@ LIB_PATH = PKG_DIR / "libmxgg.so"
 HOST_PATH = PKG_DIR / "_mxgg_host.so"
 
 SOURCES = ["capi.hip", "quant.hip", "swiglu.hip", "route.hip", "groups.hip", "gemm.hip"]
-HEADERS = ["mxgg_internal.h", "mx_device.h", "gemm_thin.h"]
+HEADERS = ["mxgg_internal.h", "mx_device.h", "gemm_thin.h", "wgrad_ahead.h"]
 
 ARCH = os.environ.get("MXGG_OFFLOAD_ARCH", "gfx950")
 
