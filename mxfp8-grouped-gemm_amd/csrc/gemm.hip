@@ -430,7 +430,7 @@ __device__ __forceinline__ void release_barrier() {
 // after each fragment read.  Only experts whose token range is not a multiple
 // of 16 take this path.
 // AHEAD (scaled only): the caller issued the loads of the first two stages
-// itself (issue_ahead()), then at most kAheadStores stores of the tile before,
+// itself (Stream::prologue), then at most kAheadStores stores of the tile before,
 // or waited for all of it.  vmcnt retires in issue order, so the first waits
 // leave those stores in flight: they drain behind this tile's first two stages.
 template <bool SCALED, bool MASK = false, bool AHEAD = false, class SM>
