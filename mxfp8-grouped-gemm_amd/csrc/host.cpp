@@ -13,10 +13,13 @@
 // catches torch.OutOfMemoryError).
 //
 // Library functions are reached through addresses handed in once by bind(), so
-// this module does not link against libmxgg.so.
+// this module does not link against libmxgg.so; bind() refuses a library of
+// another ABI version than the header this module was compiled with.
 #include <torch/extension.h>
 
 #include <optional>
+#include <stdexcept>
+#include <string>
 #include <tuple>
 #include <variant>
 #include <vector>
@@ -43,10 +46,17 @@ struct Lib {
 Lib lib;
 
 void bind(const py::dict& address) {
+  const auto version = reinterpret_cast<decltype(&::mxgg_abi_version)>(
+      address["mxgg_abi_version"].cast<uintptr_t>())();
+  if (version != MXGG_ABI_VERSION)
+    throw std::runtime_error("built for ABI version " + std::to_string(MXGG_ABI_VERSION) +
+                             ", the library has " + std::to_string(version));
+  Lib l;
 #define MXGG_FN(name) \
-  lib.name = reinterpret_cast<decltype(lib.name)>(address["mxgg_" #name].cast<uintptr_t>());
+  l.name = reinterpret_cast<decltype(l.name)>(address["mxgg_" #name].cast<uintptr_t>());
   MXGG_FNS
 #undef MXGG_FN
+  lib = l;
 }
 
 constexpr int64_t kMaxOperandBytes = 0x7FFFFFF0;  // the C ABI's bound on (rows - 1) * ld + K

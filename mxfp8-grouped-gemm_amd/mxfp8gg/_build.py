@@ -76,7 +76,8 @@ def _host_command(out: Path) -> list[str]:
 
 def build(verbose: bool = True) -> Path:
     """Compile every HIP source for gfx950, link libmxgg.so and build the host
-    module beside it (always rebuilds)."""
+    module beside it (always rebuilds).  The library is in place also where
+    the host module does not build, which is raised last."""
     BUILD_DIR.mkdir(parents=True, exist_ok=True)
     cc = hipcc()
     objs = []
@@ -86,13 +87,14 @@ def build(verbose: bool = True) -> Path:
         objs.append(obj)
         cmds.append([cc, *HIPCC_FLAGS, "-c", str(CSRC_DIR / src), "-o", str(obj)])
     host_tmp = HOST_PATH.with_suffix(".so.tmp")
-    cmds.append(_host_command(host_tmp))
-    with _cf.ThreadPoolExecutor(max_workers=len(cmds)) as ex:
+    with _cf.ThreadPoolExecutor(max_workers=len(cmds) + 1) as ex:
+        host = ex.submit(lambda: _run(_host_command(host_tmp)))
         list(ex.map(_run, cmds))
+        tmp = LIB_PATH.with_suffix(".so.tmp")
+        _run([cc, "-shared", "-fPIC", f"--offload-arch={ARCH}", *map(str, objs), "-o", str(tmp)])
+        os.replace(tmp, LIB_PATH)
+        host.result()
     os.replace(host_tmp, HOST_PATH)
-    tmp = LIB_PATH.with_suffix(".so.tmp")
-    _run([cc, "-shared", "-fPIC", f"--offload-arch={ARCH}", *map(str, objs), "-o", str(tmp)])
-    os.replace(tmp, LIB_PATH)
     if verbose:
         print(f"[mxfp8gg] built {LIB_PATH}")
     return LIB_PATH

@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes
 import threading
+import warnings
 from pathlib import Path
 
 import torch  # noqa: F401  (its libraries back the native host module)
@@ -149,7 +150,9 @@ _native = None
 def native():
     """The native host path (csrc/host.cpp), loaded with the library: checks,
     allocations and the library call of an op in one step, for the plain case
-    of its arguments."""
+    of its arguments.  None where the module cannot be used (it is bound to
+    torch's C++ ABI, the library is not): every op then takes its Python form,
+    which calls the same kernels."""
     if _native is None:
         load()
     return _native
@@ -159,12 +162,16 @@ def _load_native(lib: ctypes.CDLL):
     import importlib.machinery
     import importlib.util
 
-    if not HOST_PATH.exists():
-        raise RuntimeError(f"{HOST_PATH} is missing: build it first (mxfp8gg._build.build())")
-    loader = importlib.machinery.ExtensionFileLoader("_mxgg_host", str(HOST_PATH))
-    mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_mxgg_host", loader))
-    loader.exec_module(mod)
-    mod.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in SIGNATURES})
+    try:
+        loader = importlib.machinery.ExtensionFileLoader("_mxgg_host", str(HOST_PATH))
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_mxgg_host", loader))
+        loader.exec_module(mod)
+        mod.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in SIGNATURES})
+    except (ImportError, RuntimeError, LookupError) as e:
+        warnings.warn(f"the native host module {HOST_PATH} cannot be used ({e}); ops take their "
+                      "Python form, with the same results and more host time per call (build it: "
+                      "mxfp8gg._build.build())", RuntimeWarning, stacklevel=3)
+        return None
     return mod
 
 

@@ -43,8 +43,8 @@ def _stream_ptr(t: torch.Tensor) -> int:
 
 def _native(x, scaling_mode="rceil"):
     """The native host path for an op on the device tensor x, or None where the
-    Python form decides (another device, an unusual mode: it converts or
-    raises)."""
+    Python form decides (no host module, another device, an unusual mode: it
+    converts or raises)."""
     if isinstance(x, torch.Tensor) and x.is_cuda and scaling_mode.__class__ is str \
             and scaling_mode in _MODES:
         return _lib.native()

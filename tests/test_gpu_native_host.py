@@ -208,3 +208,20 @@ def test_scale_types_and_torch_errors(gpu):
         _same(ops.grouped_mm(q, w, ends, s.view(same), ws.view(same)), want)
     with pytest.raises(torch.OutOfMemoryError):
         ops._dim1_native(_bf16(gpu, 64, 64), None, "rceil", cap=1 << 46)
+
+
+def test_ops_run_without_the_host_module(gpu, monkeypatch):
+    """Where the host module cannot be used (native() is None) every op takes
+    its Python form, with the same results."""
+    x, wgu, wd = _bf16(gpu, 64, 128), _bf16(gpu, 4, 256, 128), _bf16(gpu, 4, 128, 128)
+    idx = torch.arange(128, device=gpu, dtype=torch.int32).reshape(64, 2) % 4
+    leaves = [t.requires_grad_(True) for t in (x, wgu, wd)]
+
+    def step():
+        out = mxfp8gg.moe_routed_ffn(x, idx, None, wgu, wd)
+        return [out.detach(), *torch.autograd.grad(out, leaves, torch.ones_like(out))]
+
+    want = step()
+    monkeypatch.setattr(_lib, "_native", None)
+    assert _lib.native() is None
+    _same(step(), want)
