@@ -4,9 +4,11 @@ The launch takes the thin-capable kernel where the average expert has at most
 128 rows; the same groups inside a taller operand (rows past the last group
 end) take the 256-row kernel.  Every output element is the same chain of MFMAs
 in both, so the rows inside the groups must be equal bit for bit, and both are
-held against the float64 oracle.  K below, at and past the six ring stages
-makes the load stream cross tiles; N off the 128-column grid leaves a partial
-tile and an empty second half.
+held against the float64 oracle.  N off the 128-column grid leaves a partial
+tile and an empty second half.  The small launches give every workgroup at most
+one work item (their load stream crosses from a tile's first 128 columns to its
+second, with K below, at and past the six ring stages); the launches of several
+rounds cross from tile to tile and from expert to expert.
 """
 import numpy as np
 import pytest
@@ -22,7 +24,7 @@ pytestmark = pytest.mark.gpu
 
 SIZES = {
     "thin": [64, 0, 1, 60, 3, 61, 2, 64],          # starts on and off the 4-row grid
-    "mixed": [5, 65, 64, 0, 128, 1, 300, 17],      # thin runs between wide tiles
+    "mixed": [5, 65, 64, 0, 128, 1, 300, 17],      # both kinds in one launch
     "one": [33],
 }
 
@@ -87,3 +89,75 @@ def test_thin_swiglu_equals_wide(gpu, sizes, F, K, mode):
         assert torch.equal(got[1], sw[:M])
     aq, as_ = ops.swiglu_quant(h, mode)
     assert torch.equal(q.view(torch.uint8), aq.view(torch.uint8)) and torch.equal(s, as_)
+
+
+# ---------------------------------------------------------------------------
+# Several rounds of the grid: a workgroup's second and later tiles, the load
+# stream crossing from one expert's tile to another's, and the ring passing
+# between thin and 256-row tiles.
+# ---------------------------------------------------------------------------
+def _tiles(sizes, n):
+    """(256-row or thin) x 256-column tiles of a launch."""
+    beg = np.cumsum(sizes) - sizes
+    rows = np.where(np.asarray(sizes) > 0, np.asarray(sizes) + beg % 4, 0)
+    return int(((rows + 255) // 256).sum()) * ((n + 255) // 256)
+
+
+def _cus(gpu):
+    return torch.cuda.get_device_properties(gpu).multi_processor_count
+
+
+THIN_64 = [(37 * i) % 61 for i in range(64)]             # 0 .. 60 rows, all thin
+MIXED_48 = [5, 65, 64, 0, 128, 1, 300, 17] * 6
+WIDE_48 = [65 + 4 * (i % 16) for i in range(48)]         # no thin tile
+
+
+def _equals_wide(gpu, sizes, N, K, scaled, out_dtype, split):
+    a, a_s, w, w_s, ends = _case(gpu, sizes, N, K, scaled, 3)
+    big, big_s = _taller(a, a_s, len(sizes))
+    wide = ops.grouped_mm(big, w, ends, big_s, w_s, out_dtype=out_dtype, split_tail=split)
+    bits = torch.int16 if out_dtype == torch.bfloat16 else torch.int32
+    for _ in range(3):
+        y = ops.grouped_mm(a, w, ends, a_s, w_s, out_dtype=out_dtype, split_tail=split)
+        assert torch.equal(y.view(bits), wide[:a.shape[0]].view(bits))
+
+
+@pytest.mark.parametrize("out_dtype,scaled", [(torch.bfloat16, True), (torch.float32, True),
+                                              (torch.bfloat16, False)])
+@pytest.mark.parametrize("sizes,K", [
+    (THIN_64, 32),       # one stage a tile: six tiles of up to six experts in flight
+    (THIN_64, 640), (THIN_64, 2080),
+    (MIXED_48, 32), (MIXED_48, 640), (MIXED_48, 2080),
+    (WIDE_48, 640),
+])
+def test_several_rounds_equal_wide_tiles(gpu, sizes, K, out_dtype, scaled):
+    N = 4096
+    assert _tiles(sizes, N) >= 2.5 * _cus(gpu)
+    _equals_wide(gpu, sizes, N, K, scaled, out_dtype, False)
+
+
+def test_split_last_round_of_thin_tiles(gpu):
+    """33 thin experts over 16 column tiles: two whole rounds, then 16 tiles cut
+    along K, each of two thin pieces; the same tiles and ranges as in the
+    256-row kernel, so the same bits."""
+    sizes, N, K = [1 + (7 * i) % 60 for i in range(33)], 4096, 2080
+    rem = _tiles(sizes, N) % _cus(gpu)
+    assert _tiles(sizes, N) > _cus(gpu) and 0 < rem <= _cus(gpu) // 2
+    for dtype in (torch.bfloat16, torch.float32):
+        _equals_wide(gpu, sizes, N, K, True, dtype, True)
+
+
+@pytest.mark.parametrize("keep", [False, True])
+@pytest.mark.parametrize("sizes,K", [(THIN_64 * 2, 32), (THIN_64 * 2, 800), (MIXED_48 * 2, 96),
+                                     (MIXED_48 * 2, 800), (WIDE_48 * 2, 800)])
+def test_swiglu_several_rounds_equal_wide(gpu, sizes, K, keep):
+    F, E, M = 1024, len(sizes), sum(sizes)
+    assert _tiles(sizes, 2 * F) >= 2.5 * _cus(gpu)
+    a, a_s, w, w_s, ends = _case(gpu, sizes, 2 * F, K, True, 9)
+    big, big_s = _taller(a, a_s, E)
+    want = ops.grouped_mm_swiglu_quant(big, w, ends, big_s, w_s, return_h=keep)
+    for _ in range(3):
+        got = ops.grouped_mm_swiglu_quant(a, w, ends, a_s, w_s, return_h=keep)
+        for x, y in zip(got, want):
+            assert torch.equal(x.contiguous().view(torch.uint8),
+                               y[:M].contiguous().view(torch.uint8))
