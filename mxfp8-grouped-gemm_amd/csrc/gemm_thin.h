@@ -503,9 +503,23 @@ __device__ __forceinline__ void thin_run(SmemThin& sm, const FwdArgs& args, cons
   wait_barrier<0>();
 }
 
+// The kernel's first argument, read again from the kernel-argument segment.
+// Kept in registers over the tile loop, the 46 argument words of two kinds of
+// tile outnumber the scalar registers (115 spilled to vector lanes in the fp32
+// form, 73 in bf16; read per tile 38 and 39), and the 256-row tiles paid for it:
+// 32 experts of 100 rows, N 7168, K 2048, 140.3 -> 139.4 us (k_grouped_fwd
+// 138.2), with SwiGLU 150.6 -> 148.1 (148.3).
+__device__ __forceinline__ FwdArgs reread_args() {
+  typedef const FwdArgs __attribute__((address_space(4))) * KernArgs;
+  KernArgs p = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));  // opaque: the loads stay where they are
+  return *(const FwdArgs*)p;
+}
+
 // ---------------------------------------------------------------------------
 // The grouped forward for launches whose experts hold few rows: the tile order
 // and the split of k_grouped_fwd, with thin tiles for the groups that fit one.
+// `args` is the first parameter (reread_args).
 // ---------------------------------------------------------------------------
 template <bool SCALED, int OUT>
 __global__ __launch_bounds__(kThreads, 1) void k_grouped_fwd_thin(FwdArgs args, uint32_t gm) {
@@ -577,9 +591,10 @@ __global__ __launch_bounds__(kThreads, 1) void k_grouped_fwd_thin(FwdArgs args, 
     FwdItem it;
     fwd_item<SWIGLU>(sm, pl, E, K, gm, lid, it);
     if (is_thin(it.gb, it.ge)) {  // this item and the thin ones after it
-      thin_run<SCALED, OUT>(sm, args, pl, E, gm, base, it);
+      thin_run<SCALED, OUT>(sm, reread_args(), pl, E, gm, base, it);
       continue;
     }
+    const FwdArgs args = reread_args();
     Operand P, Q;
     fwd_operands<SCALED, SWIGLU, false>(args, it, P, Q);
     const uint32_t q0 = it.q0, p0 = it.p0;
