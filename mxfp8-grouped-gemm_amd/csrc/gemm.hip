@@ -1427,11 +1427,18 @@ hipError_t launch_grouped_fwd(const FwdArgs& a, hipStream_t stream) {
                   : a.swiglu_mode == MXGG_SCALE_FLOOR ? (keep ? kOutSwigluKeepFloor : kOutSwigluFloor)
                   : a.out_f32                         ? kOutF32
                                                       : kOutBf16;
-  // Thin tiles take experts of at most 64 rows.  The thin-capable kernel runs
-  // 256-row tiles up to 4% slower (its wide path shares registers with the thin
-  // one), so it is left out where the average expert has more rows than two
-  // thin tiles: 32 equal experts, N 4096, K 7168, this kernel against the other:
-  // 64 rows 179 / 190 us, 100 rows 194 / 194, 192 rows 212 / 204.
+  // Thin tiles take experts of at most 64 rows.  The sizes are on the device, so
+  // the line is drawn by the average (M counts padding and rows past the last
+  // group end): up to two thin tiles per expert the thin-capable kernel is
+  // faster where some expert is that small or rounds are partial, and level
+  // elsewhere; above, routings gain and lose.  32 experts, bf16, k_grouped_fwd /
+  // k_grouped_fwd_thin, us, at N 4096 x K 7168 and N 7168 x K 2048:
+  //   rows      equal             multinomial       Zipf(1)           one expert
+  //     64  182/178 114/104   189/191 116/112   245/217 115/110   88/72  33/31
+  //    100  197/198 140/141   198/200 140/142   244/231 141/132
+  //    128  202/202 144/144   204/206 145/145   249/241 152/143   90/90  61/58
+  //    192  213/215 157/157   221/225 157/156   277/275 152/154
+  //    400  377/379 215/218   372/376 219/218   410/412 239/245
   const bool thin = (int64_t)a.M <= 128 * (int64_t)(a.group_ends ? a.E : 1);
 #define MXGG_FWD(S, O)                                                                   \
   if (thin)                                                                              \

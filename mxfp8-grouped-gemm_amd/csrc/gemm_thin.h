@@ -42,50 +42,87 @@ static_assert(kThinRingBytes >= 2u * kStageBytes, "the ring also holds two stage
 // of a wide one.
 struct __align__(16) SmemThin {
   uint8_t ring[2][kThinRingBytes / 2];  // wide stages at ring[0], ring[1]; thin ones end to end
-  int32_t sched[kMaxGroups + 1];   // prefix of m-tiles over groups
+  int32_t order[kMaxGroups];  // first m-tile and group of every rank (order_tiles)
   int32_t gend[kMaxGroups];
-  int32_t scan_tmp[kWaves];
+  uint64_t scan_tmp[kWaves];
 };
 static_assert(sizeof(SmemThin) <= 160 * 1024, "LDS of one compute unit");
-
-// Block-wide inclusive scan of the per-group counts count(0 .. E-1) into
-// out[1..E] (LDS, out[0] = 0).  Each thread owns 4 consecutive groups; a wave
-// scans its threads' sums with lane shifts and the four wave totals meet in
-// tmp, so the whole scan costs two barriers.  Ends with a barrier.
-template <class F>
-__device__ __forceinline__ void scan_groups(const F& count, int32_t* out, int E, int32_t* tmp) {
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  int32_t loc[4];
-  int32_t sum = 0;
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int g = 4 * t + u;
-    loc[u] = g < E ? count(g) : 0;
-    sum += loc[u];
-  }
-  int32_t inc = sum;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int32_t below = __shfl_up(inc, off);
-    inc += lane >= off ? below : 0;
-  }
-  if (lane == 63) tmp[wave] = inc;
-  __syncthreads();
-  int32_t run = inc - sum;
-  for (int w = 0; w < wave; ++w) run += tmp[w];
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int g = 4 * t + u;
-    run += loc[u];
-    if (g < E) out[g + 1] = run;
-  }
-  if (t == 0) out[0] = 0;
-  __syncthreads();
-}
 
 // Rows of group [gb, ge) are tiled by 256 from its first row rounded down to 4.
 __device__ __forceinline__ uint32_t tiled_rows(int32_t gb, int32_t ge) {
   return ge > gb ? (uint32_t)(ge - (gb & ~3)) : 0u;
+}
+
+// A group of at most 64 rows fits a thin tile.  The last, partial tile of a
+// larger group stays 256 rows high: it shares its weight tile in L2 with the
+// group's other tiles, which run beside it, and tiles of different heights in
+// the same rounds leave the workgroups with the short ones waiting (32 experts
+// of 320 rows, N 4096, K 7168: 350 us, with 64-row last tiles 403).  Groups of
+// 65 to 128 rows gained nothing from a 128-row form (198 us either way).
+__device__ __forceinline__ bool is_thin(int32_t gb, int32_t ge) {
+  return tiled_rows(gb, ge) <= kThinQ;
+}
+
+// The order of the groups' m-tiles: groups of 256-row tiles first, then thin and
+// empty ones, each kind in index order.  Thin tiles draw more bandwidth per CU
+// than 256-row ones, so a 256-row tile that starts beside them late is what the
+// launch waits for: 32 experts of multinomial sizes around 56, N 7168, K 2048,
+// 119 us in index order, 111 like this, 115 with 256-row tiles only.
+// order[r] of rank r is its first m-tile << kRankBits | its group; returns the
+// number of m-tiles.  Each thread owns 4 consecutive groups; a wave scans its
+// threads' sums with lane shifts and the wave totals meet in tmp.  Three counts
+// (wide groups, their tiles, all tiles) are 21-bit fields of one sum: a launch
+// has at most 2^26 rows (operands are below 2 GiB, rows at least 32 bytes).
+constexpr int kRankBits = 10;
+constexpr uint32_t kRankGroup = (1u << kRankBits) - 1;
+static_assert(kMaxGroups <= 1 << kRankBits, "a group index fits the low bits of a rank");
+
+__device__ __forceinline__ uint32_t order_tiles(const int32_t* gend, int32_t* order, int E,
+                                                uint64_t* tmp, uint32_t& wide_groups) {
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  uint64_t loc[4], sum = 0;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int g = 4 * t + u;
+    loc[u] = 0;
+    if (g < E) {
+      int32_t b, e;
+      group_range(gend, g, b, e);
+      const uint64_t tiles = (tiled_rows(b, e) + kTileQ - 1) / kTileQ;
+      loc[u] = tiles << 42 | (is_thin(b, e) ? 0u : tiles << 21 | 1u);
+    }
+    sum += loc[u];
+  }
+  uint64_t inc = sum;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint64_t below = __shfl_up((unsigned long long)inc, off);
+    inc += lane >= off ? below : 0;
+  }
+  if (lane == 63) tmp[wave] = inc;
+  __syncthreads();
+  uint64_t run = inc - sum, all = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    if (w < wave) run += tmp[w];
+    all += tmp[w];
+  }
+  constexpr uint32_t kField = (1u << 21) - 1;
+  const uint32_t wide = (uint32_t)all & kField, wide_tiles = (uint32_t)(all >> 21) & kField;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int g = 4 * t + u;
+    const uint32_t wg = (uint32_t)run & kField, wt = (uint32_t)(run >> 21) & kField;
+    const uint32_t at = (uint32_t)(run >> 42);
+    const bool w = ((uint32_t)loc[u] & 1u) != 0;
+    if (g < E)
+      order[w ? wg : wide + (uint32_t)g - wg] =
+          (int32_t)((w ? wt : wide_tiles + at - wt) << kRankBits | (uint32_t)g);
+    run += loc[u];
+  }
+  __syncthreads();
+  wide_groups = (uint32_t)uniform((int32_t)wide);
+  return (uint32_t)uniform((int32_t)(all >> 42));
 }
 
 // The work of one launch, the same for every workgroup.
@@ -94,6 +131,7 @@ struct FwdPlan {
   uint32_t pieces;              // thin P tiles per P tile: 2, or 1 if all tiles are thin
   uint32_t total, full;         // tiles; those in full rounds of the grid
   uint32_t S, chunk;            // K-ranges of a tile past `full`, stages per range
+  uint32_t thin_rows;           // groups of at most this many rows take thin tiles
   uint32_t items;               // work items: full tiles, then (tile, range) pairs
 };
 
@@ -106,12 +144,19 @@ struct FwdItem {
 };
 
 // Item index handled by this workgroup in the round starting at `base`
-// (>= items: none): each XCD takes a contiguous slice of the round, a last,
-// partial round included.
+// (0xFFFFFFFF: none): each XCD takes a contiguous slice of the round.  A last,
+// partial round is spread over all XCDs, and after a full round over the other
+// end of each one's workgroups: the first ones may have had a 256-row tile
+// (40 experts, one of 984 rows, the others of 24, N 3072, K 3072: 105 -> 95 us).
 __device__ __forceinline__ uint32_t fwd_lid(uint32_t base, uint32_t items) {
-  const uint32_t per = min(gridDim.x, (items - base + 7u) & ~7u) >> 3;
-  const uint32_t slot = blockIdx.x >> 3;
-  return slot < per ? base + (blockIdx.x & 7u) * per + slot : 0xFFFFFFFFu;
+  const uint32_t xcd = blockIdx.x & 7u;
+  uint32_t per = gridDim.x >> 3, slot = blockIdx.x >> 3;
+  if (items - base < gridDim.x) {
+    if (base != 0) slot = per - 1u - slot;
+    per = (items - base + 7u) >> 3;
+    if (slot >= per) return 0xFFFFFFFFu;
+  }
+  return base + xcd * per + slot;
 }
 
 template <bool SWIGLU>
@@ -131,24 +176,14 @@ __device__ __forceinline__ void fwd_item(const SmemThin& sm, const FwdPlan& pl, 
   }
   uint32_t mt, nt;
   band_decode(tile, pl.m_tiles, pl.n_tiles, gm, mt, nt);
-  // group of m-tile mt: last g with sched[g] <= mt
-  it.g = (uint32_t)last_le(sm.sched, E, mt);
+  // group of m-tile mt: the last rank whose first m-tile is <= mt
+  const uint32_t rank = (uint32_t)uniform(sm.order[last_le(sm.order, E, mt << kRankBits | kRankGroup)]);
+  it.g = rank & kRankGroup;
   group_range(sm.gend, (int)it.g, it.gb, it.ge);
   it.gb = uniform(it.gb);
   it.ge = uniform(it.ge);
-  const int32_t first = uniform(sm.sched[it.g]);
-  it.q0 = (uint32_t)(it.gb & ~3) + (mt - (uint32_t)first) * kTileQ;
+  it.q0 = (uint32_t)(it.gb & ~3) + (mt - (rank >> kRankBits)) * kTileQ;
   it.p0 = nt * pl.pieces * (SWIGLU ? kThinP / 2u : kThinP);
-}
-
-// A group of at most 64 rows takes thin tiles.  The last, partial tile of a
-// larger group stays 256 rows high: it shares its weight tile in L2 with the
-// group's other tiles, which run beside it, and tiles of different heights in
-// the same rounds leave the workgroups with the short ones waiting (32 experts
-// of 320 rows, N 4096, K 7168: 350 us, with 64-row last tiles 403).  Groups of
-// 65 to 128 rows gained nothing from a 128-row form (198 us either way).
-__device__ __forceinline__ bool is_thin(int32_t gb, int32_t ge) {
-  return tiled_rows(gb, ge) <= kThinQ;
 }
 
 // THIN: the second half of the tile's P rows starts at tile row 64.
@@ -380,7 +415,7 @@ __device__ __forceinline__ void thin_run(SmemThin& sm, const FwdArgs& args, cons
     const uint32_t lid = fwd_lid(b, pl.items);
     if (lid >= pl.items) return false;
     fwd_item<SWIGLU>(sm, pl, E, K, gm, lid, x);
-    return is_thin(x.gb, x.ge);
+    return tiled_rows(x.gb, x.ge) <= pl.thin_rows;
   };
 
   uint8_t* const ring = &sm.ring[0][0];
@@ -536,15 +571,9 @@ __global__ __launch_bounds__(kThreads, 1) void k_grouped_fwd_thin(FwdArgs args, 
   else if (threadIdx.x == 0)
     sm.gend[0] = M;
   __syncthreads();
-  scan_groups(
-      [&](int g) {
-        int32_t b, e;
-        group_range(sm.gend, g, b, e);
-        return (int32_t)((tiled_rows(b, e) + kTileQ - 1) / kTileQ);
-      },
-      sm.sched, E, sm.scan_tmp);
   FwdPlan pl;
-  pl.m_tiles = (uint32_t)uniform(sm.sched[E]);
+  uint32_t wide;  // groups of more rows than a thin tile
+  pl.m_tiles = order_tiles(sm.gend, sm.order, E, sm.scan_tmp, wide);
   // SWIGLU: N = 2F weight rows; a tile covers 128 features of a (F % 128 == 0)
   pl.n_tiles = SWIGLU ? (uint32_t)args.N / 256u : ((uint32_t)args.N + kTileP - 1) / kTileP;
   pl.total = pl.m_tiles * pl.n_tiles;
@@ -570,15 +599,22 @@ __global__ __launch_bounds__(kThreads, 1) void k_grouped_fwd_thin(FwdArgs args, 
   }
   pl.items = pl.S > 1 ? pl.full + rem * pl.S : pl.total;
   pl.pieces = 2;
+  // No thin tiles where they share a last round that is nearly full with 256-row
+  // ones and the contraction is long, or the only round is nearly full: there
+  // the 256-row tiles decide when the launch ends, and beside thin ones they
+  // take longer (two rounds of 32 experts, N 4096, K 7168: multinomial sizes
+  // around 56 180 us, with thin tiles 185; two experts of more than 64 rows 171
+  // and 184; one round of 8 experts, N 7168, K 2048: 28.0 and 30.5).  The SwiGLU
+  // forms gain from thin tiles there too (64 experts of Zipf sizes around 16,
+  // N 2048, K 2048: 67 -> 56): their 256-row epilogue is the longer one.
+  pl.thin_rows = kThinQ;
+  const bool full_round = rem == 0 || 5 * rem > 4 * G;
+  if (!SWIGLU && wide != 0 && pl.S == 1 && full_round &&
+      (nst > 40 || (nst >= 16 && pl.total <= G)))
+    pl.thin_rows = 0;
   // Nothing split and every tile thin (decode): the thin P tiles are the work
   // items, so that the last round is a finer share of the whole.
-  int wide = 0;
-  for (int g = threadIdx.x; g < E; g += kThreads) {
-    int32_t b, e;
-    group_range(sm.gend, g, b, e);
-    wide |= !is_thin(b, e);
-  }
-  if (__syncthreads_or(wide) == 0 && pl.S == 1) {
+  if (wide == 0 && pl.S == 1) {
     pl.pieces = 1;
     pl.n_tiles = ((uint32_t)args.N + kThinP - 1) / kThinP;
     pl.items = pl.total = pl.full = pl.m_tiles * pl.n_tiles;
@@ -590,7 +626,7 @@ __global__ __launch_bounds__(kThreads, 1) void k_grouped_fwd_thin(FwdArgs args, 
     if (lid >= pl.items) break;
     FwdItem it;
     fwd_item<SWIGLU>(sm, pl, E, K, gm, lid, it);
-    if (is_thin(it.gb, it.ge)) {  // this item and the thin ones after it
+    if (tiled_rows(it.gb, it.ge) <= pl.thin_rows) {  // this item and the thin ones after it
       thin_run<SCALED, OUT>(sm, reread_args(), pl, E, gm, base, it);
       continue;
     }

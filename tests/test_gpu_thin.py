@@ -136,6 +136,38 @@ def test_several_rounds_equal_wide_tiles(gpu, sizes, K, out_dtype, scaled):
     _equals_wide(gpu, sizes, N, K, scaled, out_dtype, False)
 
 
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("sizes,N,K", [
+    # both kinds where a nearly full last round leaves the thin tiles out: whole
+    # rounds of a long contraction, and the only round
+    ([5, 65] * 16, 4096, 5280), ([5, 65, 20, 64, 1, 70, 33, 66], 7168, 2080),
+    # every group index: 1024 groups, empty, thin and larger ones in any order
+    ([(7 * i) % 5 + (70 if i % 97 == 3 else 0) for i in range(1024)], 128, 96),
+    ([0] * 1000 + [66, 3, 0, 300] * 6, 300, 160),
+])
+def test_mixed_orders_equal_wide_tiles(gpu, sizes, N, K, out_dtype):
+    _equals_wide(gpu, sizes, N, K, True, out_dtype, False)
+
+
+def test_split_last_round_of_both_kinds(gpu):
+    """The split cuts other tiles than in the 256-row kernel (groups of 256-row
+    tiles come first), so sums differ by their order: fp32 sums of K products in
+    two orders differ by at most 2 K 2^-24 times the sum of their magnitudes."""
+    sizes, N, K = [30, 66, 0, 64, 5, 80, 1, 300, 17, 2, 40] * 3, 4096, 2080
+    rem = _tiles(sizes, N) % _cus(gpu)
+    assert _tiles(sizes, N) > _cus(gpu) and 0 < rem <= _cus(gpu) // 2
+    a, a_s, w, w_s, ends = _case(gpu, sizes, N, K, True, 3)
+    y = ops.grouped_mm(a, w, ends, a_s, w_s, out_dtype=torch.float32, split_tail=True)
+    whole = ops.grouped_mm(a, w, ends, a_s, w_s, out_dtype=torch.float32, split_tail=False)
+    size = ops.grouped_mm((a.view(torch.uint8) & 0x7F).view(a.dtype),
+                          (w.view(torch.uint8) & 0x7F).view(w.dtype), ends, a_s, w_s,
+                          out_dtype=torch.float32, split_tail=False)
+    assert ((y.double() - whole.double()).abs() <= 2 * K * 2.0 ** -24 * size.double()).all()
+    for _ in range(3):   # the same bits on every call
+        again = ops.grouped_mm(a, w, ends, a_s, w_s, out_dtype=torch.float32, split_tail=True)
+        assert torch.equal(again, y)
+
+
 def test_split_last_round_of_thin_tiles(gpu):
     """33 thin experts over 16 column tiles: two whole rounds, then 16 tiles cut
     along K, each of two thin pieces; the same tiles and ranges as in the
