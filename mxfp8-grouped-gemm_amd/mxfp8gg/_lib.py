@@ -40,6 +40,7 @@ OFFS_SIZES = 1
 OFFS_AUTO = 2
 
 ABI_VERSION = 13
+MAX_GROUPS = 1024  # groups of one call
 
 _P = ctypes.c_void_p
 _I64 = ctypes.c_int64

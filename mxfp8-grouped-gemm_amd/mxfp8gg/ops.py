@@ -498,10 +498,17 @@ def _weight_t_views(qt: torch.Tensor, st: torch.Tensor, E: int, N: int, K: int):
 
 # Weights of at most this many elements are cast as one run of rows: N % 32 == 0,
 # so no block of 32 rows straddles two experts, and the group table (three small
-# launches, 6 us on the device and 15 on the host) is not needed.  The large
-# casts run faster with it all the same (32 x 4096 x 7168: 747 us with the table
-# and its launches, 768 without).
+# launches, 6 us on the device and 15 on the host) is not needed.  With the table
+# and its launches / as one run, us, both casts and the one along N: 2^25
+# elements 33/22 and 27/17, 2^27 122/115 and 75/65, 2^28 215/215 and 173/164; the
+# large casts run faster with the table (32 x 4096 x 7168: 747/768 for both).
 _UNGROUPED_WEIGHT = 1 << 28
+
+
+def _one_run(w: torch.Tensor) -> bool:
+    """Whether expert weights are cast as one run of rows.  More experts than a
+    call takes groups stay with the grouped form, which refuses them."""
+    return w.numel() <= _UNGROUPED_WEIGHT and w.shape[0] <= _lib.MAX_GROUPS
 
 
 def quant_weight_dual(w: torch.Tensor, scaling_mode="rceil"):
@@ -516,7 +523,7 @@ def quant_weight_dual(w: torch.Tensor, scaling_mode="rceil"):
         raise ValueError(f"N={N} must be a multiple of 32 for MXFP8 blocks along N")
     w2 = w.reshape(E * N, K)
     r = None
-    if w.numel() <= _UNGROUPED_WEIGHT:
+    if _one_run(w):
         r = _dual_native(w2, None, scaling_mode, padded_token_capacity(E * N, E))
     q, s, qt, st, _ = r if r is not None else \
         to_mxfp8_dual(w2, _expert_ends(E, N, w.device), scaling_mode)
@@ -1160,7 +1167,7 @@ def quant_weight_for_dgrad(w: torch.Tensor, scaling_mode="rceil"):
         raise ValueError(f"N={N} must be a multiple of 32 for MXFP8 blocks along N")
     w2 = w.reshape(E * N, K)
     r = None
-    if w.numel() <= _UNGROUPED_WEIGHT:
+    if _one_run(w):
         r = _dim1_native(w2, None, scaling_mode, cap=padded_token_capacity(E * N, E))
     qt, st, _ = r if r is not None else \
         to_mxfp8_dim1(w2, _expert_ends(E, N, w.device), scaling_mode)

@@ -225,3 +225,13 @@ def test_ops_run_without_the_host_module(gpu, monkeypatch):
     monkeypatch.setattr(_lib, "_native", None)
     assert _lib.native() is None
     _same(step(), want)
+
+
+def test_more_experts_than_groups_stay_refused(gpu, monkeypatch):
+    """The weight casts take as many experts as a GEMM call takes groups, with
+    or without the group table."""
+    w = _bf16(gpu, 1024, 32, 32)
+    for cast in (ops.quant_weight_dual, ops.quant_weight_for_dgrad):
+        _same(*_both(monkeypatch, lambda: cast(w)))
+        with pytest.raises(ValueError, match="num_groups"):
+            cast(_bf16(gpu, 1025, 32, 32))
