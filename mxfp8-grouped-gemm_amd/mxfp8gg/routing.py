@@ -146,7 +146,7 @@ def gather_to_mxfp8_dual(x: torch.Tensor, plan: RoutePlan, scaling_mode="rceil",
     read straight from token order.  Returns (q, s, qt, st, offs_pad) like
     to_mxfp8_dual(gather_rows(x, plan, row_scale), plan.offs)."""
     host = _native(x, scaling_mode)
-    if host is not None and _tensors(row_scale) and x.shape[0] == plan.tokens:
+    if host is not None and _tensors(row_scale) and x.dim() == 2 and x.shape[0] == plan.tokens:
         r = host.gather_dual(x, plan.src, plan.offs, plan.topk, row_scale, _MODES[scaling_mode],
                              _stream_ptr(x))
         if _took(r, "gather_quant_dual"):

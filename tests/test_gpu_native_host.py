@@ -235,3 +235,11 @@ def test_more_experts_than_groups_stay_refused(gpu, monkeypatch):
         _same(*_both(monkeypatch, lambda: cast(w)))
         with pytest.raises(ValueError, match="num_groups"):
             cast(_bf16(gpu, 1025, 32, 32))
+
+
+def test_gather_of_a_scalar_is_a_type_error(gpu):
+    plan = routing.route_plan(torch.zeros((4, 1), dtype=torch.int32, device=gpu), 2)
+    for gather in (routing.gather_to_mxfp8_dual, routing.gather_to_mxfp8_dim0):
+        for x in (_bf16(gpu), _bf16(gpu, 4)):
+            with pytest.raises(TypeError):
+                gather(x, plan)
