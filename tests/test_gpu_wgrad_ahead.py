@@ -45,3 +45,58 @@ def test_boundary_inside_a_block_is_nan(gpu):
     ends = torch.tensor([40, 128, 256], dtype=torch.int32, device=gpu)
     dw = ops.grouped_wgrad(q, q, ends, s, s, out_dtype=torch.bfloat16, split_tokens=0)
     assert dw[:2].isnan().all() and (dw[2] == 128.0).all()
+
+
+# ---------------------------------------------------------------------------
+# Several rounds of the grid: the stores of a tile stay in flight behind the
+# next tile's loads from a workgroup's second tile on.
+# ---------------------------------------------------------------------------
+def _operands(gpu, sizes, n, k):
+    g = torch.Generator(device=gpu).manual_seed(n + k + len(sizes))
+    rows = sum(sizes)
+    ends = torch.tensor(np.cumsum(sizes), dtype=torch.int32, device=gpu)
+    dy = torch.randn((rows, (n + 31) // 32 * 32), generator=g, device=gpu).to(torch.bfloat16)
+    x = torch.randn((rows, (k + 31) // 32 * 32), generator=g, device=gpu).to(torch.bfloat16)
+    go, gos, pad = ops.to_mxfp8_dim1(dy, ends)
+    ia, ias, _ = ops.to_mxfp8_dim1(x, ends)
+    return go[:n], gos[:n], ia[:k], ias[:k], pad
+
+
+@pytest.mark.parametrize("n,k", [(2048, 1024),     # every wave inside dW
+                                 (2000, 1032)])    # guarded waves beside interior ones
+@pytest.mark.parametrize("sizes", [
+    [64] * 32, [128] * 32,            # one stage
+    [200] * 32, [256] * 32,           # two, or three where the start is off the 128-token grid
+    [385] * 32, [640] * 32,           # three to six
+    [200, 256, 385, 640, 33, 128, 100, 500] * 4,
+    [640, 0, 31, 128, 0, 256, 7, 500] * 4,          # empty experts last, without loads
+    [700] + [0] * 15 + [90] * 16,
+])
+def test_several_rounds_equal_rounded_fp32(gpu, sizes, n, k):
+    tiles = len(sizes) * ((n + 255) // 256) * ((k + 255) // 256)
+    assert tiles >= 3 * torch.cuda.get_device_properties(gpu).multi_processor_count
+    go, gos, ia, ias, pad = _operands(gpu, sizes, n, k)
+    want = ops.grouped_wgrad(go, ia, pad, gos, ias, out_dtype=torch.float32, split_tokens=0)
+    out = torch.full((len(sizes), n, k), 7.0, dtype=torch.bfloat16, device=gpu)
+    for _ in range(3):
+        ops.grouped_wgrad(go, ia, pad, gos, ias, out=out, out_dtype=torch.bfloat16, split_tokens=0)
+        assert torch.equal(out.view(torch.int16), want.to(torch.bfloat16).view(torch.int16))
+
+
+@pytest.mark.parametrize("at", [0, 7, 30])
+def test_nan_experts_between_full_ones(gpu, at):
+    """A boundary inside a 32-token block: both experts at it are NaN, without
+    loads, among experts of several stages in the same workgroups."""
+    n, k, sizes = 2048, 1024, [300, 160, 512, 96] * 8
+    go, gos, ia, ias, pad = _operands(gpu, sizes, n, k)
+    ends = pad.as_subclass(torch.Tensor).clone()
+    ends[at] += 8
+    want = ops.grouped_wgrad(go, ia, ends, gos, ias, out_dtype=torch.float32, split_tokens=0)
+    out = torch.full((len(sizes), n, k), 7.0, dtype=torch.bfloat16, device=gpu)
+    for _ in range(3):
+        ops.grouped_wgrad(go, ia, ends, gos, ias, out=out, out_dtype=torch.bfloat16,
+                          split_tokens=0)
+        nan = out.isnan().flatten(1)
+        assert nan[at:at + 2].all() and not nan[:at].any() and not nan[at + 2:].any()
+        keep = [e for e in range(len(sizes)) if e not in (at, at + 1)]
+        assert torch.equal(out[keep], want[keep].to(torch.bfloat16))
