@@ -70,8 +70,13 @@ constexpr int64_t kPartialBytes = 256 * 256 * 4;
 // work item i at kWgHdrBytes + i * kPartialBytes.
 constexpr int64_t kWgHdrBytes = 32768;
 // Store instructions of one wave for a tile that lies inside dW, in the weight
-// gradient whose stores overlap the next tile (two per P half and Q fragment).
-constexpr int kAheadStores = 32;
+// gradient whose stores overlap the next tile: store_bf16_direct's loops, two
+// rows of chunks per P half and Q fragment.
+constexpr uint32_t kDirectFrags = 8, kDirectHalves = 2, kDirectRows = 2;
+constexpr int kAheadStores = kDirectFrags * kDirectHalves * kDirectRows;
+// Loads of one wave for one stage: 16 of data, then 2 of scales.
+constexpr int kStageLoads = 16, kScaleLoads = 2;
+static_assert(kStageLoads + kScaleLoads + kAheadStores <= 63, "vmcnt counts to 63");
 
 struct __align__(16) Smem {
   uint8_t ring[2][kStageBytes];
@@ -430,9 +435,11 @@ __device__ __forceinline__ void release_barrier() {
 // after each fragment read.  Only experts whose token range is not a multiple
 // of 16 take this path.
 // AHEAD (scaled only): the caller issued the loads of the first two stages
-// itself (Stream::prologue), then at most kAheadStores stores of the tile before,
+// itself (Stream::prologue), then exactly kAheadStores stores of the tile before,
 // or waited for all of it.  vmcnt retires in issue order, so the first waits
 // leave those stores in flight: they drain behind this tile's first two stages.
+// With fewer stores the counts would reach into the loads; more vector-memory
+// instructions (a spill) only make them stricter.
 template <bool SCALED, bool MASK = false, bool AHEAD = false, class SM>
 __device__ __forceinline__ void mainloop(SM& sm, const Operand& P, const Operand& Q,
                                          uint32_t klo, uint32_t kend, v4f (&acc)[64]) {
@@ -447,13 +454,13 @@ __device__ __forceinline__ void mainloop(SM& sm, const Operand& P, const Operand
   st.init(P, Q, klo, kend);
   FragAddr fa;
   fa.init();
-  // Prologue: all of stage 0 and the data of stage 1 (its scales follow in
-  // the first stage), then publish stage 0 and read the part of it that the
-  // loop reads one stage ahead.
+  // Prologue: all of stage 0 and, if there is one, of stage 1 (issued here or by
+  // the caller), then publish stage 0 and read the part of it that the loop
+  // reads one stage ahead.
   if constexpr (!AHEAD) st.prologue(sm.ring[0], sm.ring[1], P, Q, kbeg, nst);
   constexpr int kLeft = AHEAD ? kAheadStores : 0;
   if (nst > 1)
-    wait_barrier<(SCALED ? 18 : 16) + kLeft>();
+    wait_barrier<kStageLoads + (SCALED ? kScaleLoads : 0) + kLeft>();
   else
     wait_barrier<kLeft>();
   MXGG_FENCE();

@@ -17,9 +17,9 @@
 // and Q fragment 4H + j, columns 64G + 16g .. +15 of row 64H + 4c + j (of the
 // wave's 128 x 128): two 16-byte chunks.  Lanes c and c ^ 1 swap one chunk, so
 // that one instruction writes the even lane's row and the next the odd lane's:
-// 8 rows x 128 bytes each.  Returns with at most kAheadStores stores in flight,
-// or none where the wave's block is not wholly inside dW (the guarded stores'
-// number varies).
+// 8 rows x 128 bytes each.  Issues exactly kAheadStores stores, or returns with
+// none in flight where the wave's block is not wholly inside dW (the guarded
+// stores' number varies).
 __device__ __forceinline__ void store_bf16_direct(const v4f (&acc)[64], char* out,
                                                   int64_t ldo_bytes, uint32_t q0, uint32_t qend,
                                                   uint32_t p0, uint32_t pend) {
@@ -37,9 +37,9 @@ __device__ __forceinline__ void store_bf16_direct(const v4f (&acc)[64], char* ou
       (int)(127u * (uint32_t)ldo_bytes + 256u), 0x00020000);
   const uint32_t voff = row * (uint32_t)ldo_bytes + 2u * col;
 #pragma unroll
-  for (uint32_t qj = 0; qj < 8; ++qj)
+  for (uint32_t qj = 0; qj < kDirectFrags; ++qj)
 #pragma unroll
-    for (uint32_t G = 0; G < 2; ++G) {
+    for (uint32_t G = 0; G < kDirectHalves; ++G) {
       const uint32_t a0 = 32u * G + qj;
       uint32_t x[2][4];
 #pragma unroll
@@ -59,6 +59,7 @@ __device__ __forceinline__ void store_bf16_direct(const v4f (&acc)[64], char* ou
       }
       const uint32_t r0 = 64u * (qj >> 2) + (qj & 3u);
       if (interior) {
+        static_assert(kDirectRows == 2, "the two stores below");
         const uint32_t soff = r0 * (uint32_t)ldo_bytes + 128u * G;
         __builtin_amdgcn_raw_buffer_store_b128(even, dst, voff, soff, kCacheNT);
         __builtin_amdgcn_raw_buffer_store_b128(other, dst, voff, soff + 4u * (uint32_t)ldo_bytes,
@@ -66,7 +67,7 @@ __device__ __forceinline__ void store_bf16_direct(const v4f (&acc)[64], char* ou
         continue;
       }
 #pragma unroll
-      for (uint32_t k = 0; k < 2; ++k) {
+      for (uint32_t k = 0; k < kDirectRows; ++k) {
         const u32x4 v = k ? other : even;
         const uint32_t q = qw + r0 + row + 4u * k, p = pw + 64u * G + col;
         if (q >= qend || p >= pend) continue;
