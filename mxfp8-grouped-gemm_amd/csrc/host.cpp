@@ -38,8 +38,7 @@ struct Lib {
   MXGG_FN(quant_dim0) MXGG_FN(quant_dim1) MXGG_FN(quant_dual) MXGG_FN(zero_rows_past_groups) \
   MXGG_FN(grouped_fwd) MXGG_FN(grouped_fwd_split) MXGG_FN(grouped_fwd_swiglu_quant)          \
   MXGG_FN(grouped_fwd_swiglu_quant_keep_h) MXGG_FN(grouped_wgrad) MXGG_FN(swiglu_bwd_quant)  \
-  MXGG_FN(gather_quant_dual) MXGG_FN(gather_quant_dim0) MXGG_FN(combine)                     \
-  MXGG_FN(combine_score_grad)
+  MXGG_FN(gather_quant_dual) MXGG_FN(gather_quant_dim0) MXGG_FN(combine)
   MXGG_FNS
 #undef MXGG_FN
 };
