@@ -1481,14 +1481,19 @@ hipError_t launch_grouped_wgrad(const WgradArgs& a, hipStream_t stream) {
   const dim3 grid(persistent_grid()), block(kThreads);
   const uint32_t gm = 4;
 #define MXGG_WG(S, F) hipLaunchKernelGGL((k_grouped_wgrad<S, F>), grid, block, 0, stream, a, gm)
-  // Up to 768 tokens per expert (M counts the padding) the tiles whose stores
-  // overlap the next tile's loads are faster, above they are level to 3%
-  // slower (a tile's store is then a small part of it, and the MFMAs of other
-  // CUs cover it).  32 experts, bf16 dW, k_grouped_wgrad against
-  // k_grouped_wgrad_ahead, us, tokens per expert:
-  //                      32       128       250       512        1000       2048
-  //   7168 x 2048   216/166   218/166   254/211   331/286    539/555    831/848
-  //   4096 x 7168   378/316   431/324   506/421   654/573  1062/1001  1630/1583
+  // The tiles whose stores overlap the next tile's loads, up to 768 tokens per
+  // expert.  M is the padded capacity, so the line is at about 736 tokens, 704
+  // where a routing plan padded them first.  There it is where the first of the
+  // measured shapes stops gaining: above it N 7168, K 2048 loses up to 4% over 32
+  // experts, and most others still gain.  bf16 dW, k_grouped_wgrad /
+  // k_grouped_wgrad_ahead, us:
+  //   tokens                    64      512      736      1000       2048
+  //   7168 x 2048, 32 equal   209/161  330/288  413/376  547/549   822/828
+  //                Zipf(1)    210/173  348/313  405/371  556/550   869/856
+  //           one holds all 183/185  299/304  367/370  474/482   800/807
+  //   4096 x 7168, 32 equal   431/324  645/565  865/815 1062/1019 1608/1553
+  //   7168 x 2048,  8 equal            91/85   112/101  128/117   199/189
+  //   2048 x 1024, 64 Zipf(1)         138/127  173/163  208/198   435/424
   // dW rows off the 16-byte grid would all take the guarded stores.
   constexpr int64_t kAheadTokens = 768;
   const bool ahead = a.scaled && !a.out_f32 && a.split <= 0 &&
