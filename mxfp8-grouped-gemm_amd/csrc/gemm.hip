@@ -1491,7 +1491,7 @@ hipError_t launch_grouped_wgrad(const WgradArgs& a, hipStream_t stream) {
   //   7168 x 2048, 32 equal   209/161  330/288  413/376  547/549   822/828
   //                Zipf(1)    210/173  348/313  405/371  556/550   869/856
   //           one holds all 183/185  299/304  367/370  474/482   800/807
-  //   4096 x 7168, 32 equal   431/324  645/565  865/815 1062/1019 1608/1553
+  //   4096 x 7168, 32 equal   450/317  645/565  865/815 1062/1019 1608/1553
   //   7168 x 2048,  8 equal            91/85   112/101  128/117   199/189
   //   2048 x 1024, 64 Zipf(1)         138/127  173/163  208/198   435/424
   // dW rows off the 16-byte grid would all take the guarded stores.

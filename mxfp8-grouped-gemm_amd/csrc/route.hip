@@ -460,13 +460,16 @@ hipError_t launch_combine(const uint16_t* y, int64_t ldy, int64_t yrows, const i
                           int64_t ldo, hipStream_t stream) {
   if (tokens == 0 || cols == 0) return hipSuccess;
   // A row is split into whole trips of the kernel (kCombineChunks * 64 chunks)
-  // until the launch has this many waves (top-8 rows of 7168: 64 tokens 16.5 ->
-  // 6.3 us, 1000 tokens 32 -> 27, 1900 level; splitting a row of one trip only
-  // reads perm twice: 1000 rows of 1024, 7.5 -> 8.7).
-  constexpr int64_t kCombineWaves = 4096;
+  // until the launch has as many waves as the chip holds of it at once, three per
+  // SIMD; the general loop of more slots gains a little beyond.  Top-8 rows of
+  // 7168, whole / split, us: 100 tokens 15.9/6.7, 1000 27.2/22.8, 1500 34.1/32.4;
+  // at 1700 a split in two makes a second, short round: 37.2/37.8, rows of 4096
+  // 21.3/22.7.  Top-12, 1000 and 1900 tokens: 73/37, 117/108.  Splitting a row of
+  // one trip only reads perm twice: 1000 rows of 1024, 7.5/8.7.
+  const int64_t waves = topk <= kCombineSlots ? 3072 : 4096;
   constexpr int kTrip = 64 * kCombineChunks;
   const int chunks = (int)(cols / 8), trips = (chunks + kTrip - 1) / kTrip;
-  const int64_t want = std::max<int64_t>(1, std::min<int64_t>(trips, kCombineWaves / tokens));
+  const int64_t want = std::max<int64_t>(1, std::min<int64_t>(trips, waves / tokens));
   const int per = (int)((trips + want - 1) / want) * kTrip;
   const dim3 grid((unsigned)((tokens + 3) / 4), (unsigned)((chunks + per - 1) / per));
   if (scores != nullptr)

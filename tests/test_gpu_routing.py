@@ -197,7 +197,7 @@ def test_combine_matches_oracle(gpu, scaled, T, K, E, H):
     assert np.array_equal(bits(got), ref)
 
 
-@pytest.mark.parametrize("T", [1, 5, 1025])
+@pytest.mark.parametrize("T", [1, 5, 1025, 1536, 1537])
 @pytest.mark.parametrize("K,E,H", [(8, 16, 2048), (8, 16, 2056), (3, 5, 7168), (9, 12, 4104)])
 def test_combine_of_split_rows(gpu, T, K, E, H):
     # few tokens: a row is spread over workgroups in pieces of 2048 columns
