@@ -505,10 +505,10 @@ def _weight_t_views(qt: torch.Tensor, st: torch.Tensor, E: int, N: int, K: int):
 _UNGROUPED_WEIGHT = 1 << 28
 
 
-def _one_run(w: torch.Tensor) -> bool:
+def _one_run(E: int, N: int, K: int) -> bool:
     """Whether expert weights are cast as one run of rows.  More experts than a
     call takes groups stay with the grouped form, which refuses them."""
-    return w.numel() <= _UNGROUPED_WEIGHT and w.shape[0] <= _lib.MAX_GROUPS
+    return E * N * K <= _UNGROUPED_WEIGHT and E <= _lib.MAX_GROUPS
 
 
 def quant_weight_dual(w: torch.Tensor, scaling_mode="rceil"):
@@ -523,7 +523,7 @@ def quant_weight_dual(w: torch.Tensor, scaling_mode="rceil"):
         raise ValueError(f"N={N} must be a multiple of 32 for MXFP8 blocks along N")
     w2 = w.reshape(E * N, K)
     r = None
-    if _one_run(w):
+    if _one_run(E, N, K):
         r = _dual_native(w2, None, scaling_mode, padded_token_capacity(E * N, E))
     q, s, qt, st, _ = r if r is not None else \
         to_mxfp8_dual(w2, _expert_ends(E, N, w.device), scaling_mode)
@@ -1167,7 +1167,7 @@ def quant_weight_for_dgrad(w: torch.Tensor, scaling_mode="rceil"):
         raise ValueError(f"N={N} must be a multiple of 32 for MXFP8 blocks along N")
     w2 = w.reshape(E * N, K)
     r = None
-    if _one_run(w):
+    if _one_run(E, N, K):
         r = _dim1_native(w2, None, scaling_mode, cap=padded_token_capacity(E * N, E))
     qt, st, _ = r if r is not None else \
         to_mxfp8_dim1(w2, _expert_ends(E, N, w.device), scaling_mode)
