@@ -177,7 +177,8 @@ __device__ __forceinline__ void fwd_item(const SmemThin& sm, const FwdPlan& pl, 
   uint32_t mt, nt;
   band_decode(tile, pl.m_tiles, pl.n_tiles, gm, mt, nt);
   // group of m-tile mt: the last rank whose first m-tile is <= mt
-  const uint32_t rank = (uint32_t)uniform(sm.order[last_le(sm.order, E, mt << kRankBits | kRankGroup)]);
+  const int at = last_le(sm.order, E, mt << kRankBits | kRankGroup);
+  const uint32_t rank = (uint32_t)uniform(sm.order[at]);
   it.g = rank & kRankGroup;
   group_range(sm.gend, (int)it.g, it.gb, it.ge);
   it.gb = uniform(it.gb);
